@@ -865,7 +865,7 @@ bool buildLBVH(rt_device_scene* s, const std::vector<uint32_t>& instPrimOffset, 
         if (ev[k]) (void)hipEventDestroy(ev[k]);
     // a 4-wide node pushes at most three children: the stack never holds more
     // than 3 (depth - 1) entries
-    if (ok && 3 * (uint64_t)s->bvh4Depth + 1 > RT_LDS_STACK + RT_SPILL_STACK) {
+    if (ok && 3 * (uint64_t)s->bvh4Depth + 1 > RT_MAX_STACK) {
         setError("BVH depth " + std::to_string(s->bvh4Depth) + " exceeds the traversal stack");
         return false;
     }

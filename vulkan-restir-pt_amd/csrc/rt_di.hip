@@ -26,6 +26,9 @@ namespace {
 #ifndef RT_WAVES_DI
 #define RT_WAVES_DI 4
 #endif
+#ifndef RT_WAVES_DI_POOL
+#define RT_WAVES_DI_POOL 4
+#endif
 
 constexpr uint32_t kSampleLight = 0, kSampleBSDF = 1;   // TestReSTIR::SampleType (Both = 2)
 constexpr uint32_t kShiftReconnection = 0, kShiftReplay = 1;
@@ -187,40 +190,49 @@ RT_DEV void randomReplay(const DevScene& S, TStack st, uint32_t sampleMode, DIRe
     if (diValid(rr)) diMerge(dst, rr, sample1f(rng));
 }
 
-// di_reservoir.glsl:223-281
-template <bool kCount>
-RT_DEV void reconnection(const DevScene& S, TStack st, DIResv& dst, const Surf& dstSurf, DIResv src, f3 wo,
-                         uint32_t& rng, TraceCounters* ctr) {
+// di_reservoir.glsl:223-281 up to the reconnection's visibility: src becomes the shifted sample, with the
+// weight it has if the ray to `to` is free. Returns whether the shift is valid, i.e. asks for that ray; otherwise
+// the weight is 0.
+RT_DEV bool shiftReconnection(const DevScene& S, const Surf& dstSurf, DIResv& src, f3 wo, f3& to) {
     DISample ss = src.s;
     Surf rc; diSurface(S, ss.isec, rc);
+    to = rc.pos;
     const float dist = distance(rc.pos, dstSurf.pos);
     const f3 wi = normalize(rc.pos - dstSurf.pos);
     const float cosTheta = -dot(rc.norm, wi);
     const float dstJacobian = fabsf(cosTheta) / square(dist);
     const float jacobian = dstJacobian / ss.jacobian;
     float dstPHat = 0.0f, dstSamplePdf = 0.0f;
-    // The shifted sample is formed before the visibility of its reconnection is traced, so that
-    // only it and the ray stay live across the traversal; an occluded shift merges with weight 0
-    // (only its M counts: a weight-0 candidate is never picked).
-    if (diSampleValid(ss) && dist > 1e-4f && cosTheta > 0.0f && !isnan(jacobian) && ss.jacobian > 0.0f) {
-        const Mat dstMat = loadMat(S, dstSurf.matIndex);
-        if (!isnan(ss.samplePdf) && ss.samplePdf > 1e-6f) {
-            const f3 Li = src.s.Li * evalBSDF(dstMat, dstSurf.albedo, dstSurf.norm, wo, wi) * satDot(dstSurf.norm, wi) /
-                          ss.samplePdf;
-            dstPHat = luminance(Li * jacobian);
-        }
-        if (ss.isLight) dstSamplePdf = luminance(rc.albedo) / S.lightTable[0].prob / dstJacobian;
-        else dstSamplePdf = evalPdf(dstMat, dstSurf.norm, wo, wi);
-        ss.jacobian = dstJacobian;
-        ss.samplePdf = dstSamplePdf;
-        if (ss.samplePdf < 1e-6f || isnan(ss.samplePdf)) ss.samplePdf = 0.0f;
-        src.s = ss;
-        src.resampleWeight *= dstPHat / src.weight;
-        if (isnan(src.resampleWeight)) src.resampleWeight = 0.0f;
-        if (!traceVisibility<kCount>(S, st, dstSurf.pos, rc.pos, ctr)) src.resampleWeight = 0.0f;
-    } else {
+    if (!(diSampleValid(ss) && dist > 1e-4f && cosTheta > 0.0f && !isnan(jacobian) && ss.jacobian > 0.0f)) {
         src.resampleWeight = 0.0f;
+        return false;
     }
+    const Mat dstMat = loadMat(S, dstSurf.matIndex);
+    if (!isnan(ss.samplePdf) && ss.samplePdf > 1e-6f) {
+        const f3 Li = src.s.Li * evalBSDF(dstMat, dstSurf.albedo, dstSurf.norm, wo, wi) * satDot(dstSurf.norm, wi) /
+                      ss.samplePdf;
+        dstPHat = luminance(Li * jacobian);
+    }
+    if (ss.isLight) dstSamplePdf = luminance(rc.albedo) / S.lightTable[0].prob / dstJacobian;
+    else dstSamplePdf = evalPdf(dstMat, dstSurf.norm, wo, wi);
+    ss.jacobian = dstJacobian;
+    ss.samplePdf = dstSamplePdf;
+    if (ss.samplePdf < 1e-6f || isnan(ss.samplePdf)) ss.samplePdf = 0.0f;
+    src.s = ss;
+    src.resampleWeight *= dstPHat / src.weight;
+    if (isnan(src.resampleWeight)) src.resampleWeight = 0.0f;
+    return true;
+}
+
+// The shifted sample is formed before the visibility of its reconnection is traced, so that only it and the ray
+// stay live across the traversal; an occluded shift merges with weight 0 (only its M counts: a weight-0 candidate
+// is never picked).
+template <bool kCount>
+RT_DEV void reconnection(const DevScene& S, TStack st, DIResv& dst, const Surf& dstSurf, DIResv src, f3 wo,
+                         uint32_t& rng, TraceCounters* ctr) {
+    f3 to;
+    if (shiftReconnection(S, dstSurf, src, wo, to) && !traceVisibility<kCount>(S, st, dstSurf.pos, to, ctr))
+        src.resampleWeight = 0.0f;
     if (diValid(src)) diMerge(dst, src, sample1f(rng));
 }
 
@@ -319,7 +331,48 @@ __global__ __launch_bounds__(kTileThreads, RT_WAVES_DI) void k_di_temporal(DevSc
     diStore(tempR, p, resv);
 }
 
-// di_spatial.glsl:9-119 and the accumulation of di_spatial.comp:21-27
+// findNeighborReservoir (di_spatial.glsl:9-34) of the disk sample drawn from rng: the neighbour's reservoir, if
+// its surface is similar and the reservoir valid.
+RT_DEV bool diNeighbor(const rt_camera& cam, const GB& g, const DIPlanes& tempR, const DIPixel& px, uint32_t& rng,
+                       DIResv& nres) {
+    const f2 texel = mk2(1.0f / (float)g.W, 1.0f / (float)g.H);
+    const f2 nb = px.uv + (toConcentricDisk(sample2f(rng)) * kDIRadius) * texel;
+    if (nb.x < 0.0f || nb.y < 0.0f || nb.x > 1.0f || nb.y > 1.0f) return false;
+    const int qx = (int)(nb.x * (float)cam.filmSize[0]);
+    const int qy = (int)(nb.y * (float)cam.filmSize[1]);
+    GPix np;
+    if (!unpackGB(texDN(g, nb), fetchAM(g, qx, qy), np)) return false;
+    const CamRay nr = pinholeRay(cam, mk2(nb.x, 1.0f - nb.y));
+    const f3 posN = nr.ori + nr.dir * (np.depth - 1e-4f);
+    if (dot(np.norm, px.gp.norm) < 0.9f || distance(px.pos, posN) > 0.4f) return false;
+    nres = diAt(tempR, cam.filmSize[0], cam.filmSize[1], qx, qy);
+    return diValid(nres);
+}
+
+// The shading of di_spatial.glsl:110-119 and the accumulation of di_spatial.comp:21-27.
+RT_DEV void diShade(const DevScene& S, const rt_camera& cam, const DIPixel& px, DIResv& resv, const DIPlanes& thisR,
+                    size_t p, float* directOut, bool surface) {
+    f3 radiance = s3(0.0f);
+    if (surface) {
+        diCap(resv, kDICap);
+        if (!diValid(resv)) diReset(resv);
+        diStore(thisR, p, resv);
+        if (diValid(resv) && diSampleValid(resv.s)) {
+            Surf sf; diSurface(S, resv.s.isec, sf);
+            const f3 wi = normalize(sf.pos - px.pos);
+            if (resv.sampleCount > 0u) {
+                const Mat mat = loadMat(S, px.surf.matIndex);
+                const f3 Li = resv.s.Li * evalBSDF(mat, px.gp.albedo, px.gp.norm, -px.ray.dir, wi) *
+                              satDot(px.gp.norm, wi) / resv.s.samplePdf;
+                if (!isBlack(Li)) radiance = Li / luminance(Li) * resv.resampleWeight / (float)resv.sampleCount;
+            }
+        }
+        radiance = clampColor(radiance);
+    }
+    accumulate(directOut, p, radiance, cam.frameIndex);
+}
+
+// di_spatial.glsl:9-119 with the replay (or hybrid) shift
 template <bool kCount, uint32_t kShift>
 __global__ __launch_bounds__(kTileThreads, RT_WAVES_DI) void k_di_spatial(DevScene S, rt_camera cam, GB g,
                                                                          rt_di_settings set, DIPlanes tempR,
@@ -330,47 +383,102 @@ __global__ __launch_bounds__(kTileThreads, RT_WAVES_DI) void k_di_spatial(DevSce
     if (x >= g.W || y >= g.H) return;
     TStack st = laneStack(stk);
     const size_t p = (size_t)y * g.W + x;
-    f3 radiance = s3(0.0f);
     DIPixel px;
-    if (diPixel(cam, g, x, y, px)) {
+    DIResv resv;
+    const bool surface = diPixel(cam, g, x, y, px);
+    if (surface) {
         uint32_t rng = makeSeedPix(cam.seed, x, y) ^ 2u;
-        const f3 wo = -px.ray.dir;
-        DIResv resv = diLoad(tempR, p);
+        resv = diLoad(tempR, p);
         if (set.spatialReuse) {
-            const f2 texel = mk2(1.0f / (float)g.W, 1.0f / (float)g.H);
             for (uint32_t i = 0; i < kDINeighbors; i++) {
-                const f2 nb = px.uv + (toConcentricDisk(sample2f(rng)) * kDIRadius) * texel;
-                // findNeighborReservoir (di_spatial.glsl:9-34)
-                if (nb.x < 0.0f || nb.y < 0.0f || nb.x > 1.0f || nb.y > 1.0f) continue;
-                const int qx = (int)(nb.x * (float)cam.filmSize[0]);
-                const int qy = (int)(nb.y * (float)cam.filmSize[1]);
-                GPix np;
-                if (!unpackGB(texDN(g, nb), fetchAM(g, qx, qy), np)) continue;
-                const CamRay nr = pinholeRay(cam, mk2(nb.x, 1.0f - nb.y));
-                const f3 posN = nr.ori + nr.dir * (np.depth - 1e-4f);
-                if (dot(np.norm, px.gp.norm) < 0.9f || distance(px.pos, posN) > 0.4f) continue;
-                const DIResv nres = diAt(tempR, cam.filmSize[0], cam.filmSize[1], qx, qy);
-                if (diValid(nres))
-                    reuseAndMerge<kCount, kShift>(S, st, set.sampleType, resv, px.surf, nres, wo, rng, ctr);
+                DIResv nres;
+                if (diNeighbor(cam, g, tempR, px, rng, nres))
+                    reuseAndMerge<kCount, kShift>(S, st, set.sampleType, resv, px.surf, nres, -px.ray.dir, rng, ctr);
             }
             visibilityCheck<kCount>(S, st, resv, px.pos, ctr);
         }
-        diCap(resv, kDICap);
-        if (!diValid(resv)) diReset(resv);
-        diStore(thisR, p, resv);
-        if (diValid(resv) && diSampleValid(resv.s)) {
-            Surf sf; diSurface(S, resv.s.isec, sf);
-            const f3 wi = normalize(sf.pos - px.pos);
-            if (resv.sampleCount > 0u) {
-                const Mat mat = loadMat(S, px.surf.matIndex);
-                const f3 Li = resv.s.Li * evalBSDF(mat, px.gp.albedo, px.gp.norm, wo, wi) * satDot(px.gp.norm, wi) /
-                              resv.s.samplePdf;
-                if (!isBlack(Li)) radiance = Li / luminance(Li) * resv.resampleWeight / (float)resv.sampleCount;
-            }
-        }
-        radiance = clampColor(radiance);
     }
-    accumulate(directOut, p, radiance, cam.frameIndex);
+    diShade(S, cam, px, resv, thisR, p, directOut, surface);
+}
+
+// di_spatial.glsl:9-119 with the reconnection shift. A shift's random numbers and M do not depend on its
+// visibility, so a tile's shifts are evaluated first, their visibility rays traced from a pool by whichever lane is
+// free, and the merges done last in the neighbours' order; the picked neighbour's shifted sample is then formed
+// again. With a ray per neighbour traced in the loop a wave ran with 15 of 64 lanes active: a lane without a valid
+// neighbour, or with a short ray, waited for the longest of the tile, ten times over (1920x1080, 1.1M triangles:
+// 3.78 -> 2.07 ms, 1.77 -> 0.80 G VALU instructions). A shift of weight 0 merges the same whether it is occluded or
+// not, so its ray is traced by the counting build only. 256 rays hold the LDS to 11 KB, 14 waves per CU.
+constexpr uint32_t kDIPoolRays = 256;
+template <bool kCount>
+__global__ __launch_bounds__(kTileThreads, RT_WAVES_DI_POOL) void k_di_spatial_pool(DevScene S, rt_camera cam, GB g,
+                                                                         rt_di_settings set, DIPlanes tempR,
+                                                                         DIPlanes thisR, float* directOut,
+                                                                         TraceCounters* ctr) {
+    __shared__ StackLDS<kTileThreads, kPoolStackWords> stk;
+    __shared__ VisibilityPool<kDIPoolRays> pool;
+    __shared__ float weights[kDINeighbors][kTileThreads];
+    PIXEL_INDEX
+    const TStack st = laneStack(stk);
+    const uint32_t lane = threadIdx.x;
+    const bool inside = x < g.W && y < g.H;
+    const size_t p = (size_t)y * g.W + x;
+    DIPixel px;
+    DIResv resv;
+    const bool surface = inside && diPixel(cam, g, x, y, px);
+    if (surface) resv = diLoad(tempR, p);
+    if (set.spatialReuse) {
+        const uint32_t rng0 = makeSeedPix(cam.seed, x, y) ^ 2u;
+        uint32_t rng = rng0, valid = 0, count = 0;
+        pool.blocked[lane] = 0u;
+        if (surface) {
+            pool.origin[0][lane] = px.pos.x; pool.origin[1][lane] = px.pos.y; pool.origin[2][lane] = px.pos.z;
+        }
+        for (uint32_t i = 0; i < kDINeighbors; i++) {
+            bool want = false;
+            f3 to = s3(0.0f);
+            DIResv nres;
+            if (surface && diNeighbor(cam, g, tempR, px, rng, nres)) {
+                (void)sample1f(rng);  // the merge's random number
+                valid |= 1u << i;
+                resv.sampleCount += nres.sampleCount;
+                want = shiftReconnection(S, px.surf, nres, -px.ray.dir, to) && (kCount || nres.resampleWeight != 0.0f);
+                weights[i][lane] = nres.resampleWeight;
+            }
+            poolAdd(pool, count, want, to, i);
+            if (count > kDIPoolRays - kTileThreads || i + 1 == kDINeighbors) poolTrace<kCount>(S, st, pool, count, ctr);
+        }
+        // merges (DIReservoirMerge): the weights' running sum and the last pick
+        bool check = false;
+        f3 to = s3(0.0f);
+        if (surface) {
+            const uint32_t blocked = pool.blocked[lane];
+            uint32_t pick = 0u;
+            bool picked = false;
+            rng = rng0;
+            for (uint32_t i = 0; i < kDINeighbors; i++) {
+                const uint32_t before = rng;
+                (void)sample2f(rng);
+                if (!((valid >> i) & 1u)) continue;
+                const float u = sample1f(rng);
+                const float w = (blocked >> i) & 1u ? 0.0f : weights[i][lane];
+                resv.resampleWeight += w;
+                if (u * resv.resampleWeight < w) { pick = before; picked = true; }
+            }
+            DIResv nres;
+            if (picked && diNeighbor(cam, g, tempR, px, pick, nres)) {
+                (void)shiftReconnection(S, px.surf, nres, -px.ray.dir, to);
+                resv.s = nres.s;
+                resv.weight = nres.weight;
+            }
+            // visibility of the final sample (di_spatial.glsl:99-108)
+            check = diValid(resv) && diSampleValid(resv.s);
+            if (check) { Surf sf; diSurface(S, resv.s.isec, sf); to = sf.pos; }
+        }
+        poolAdd(pool, count, check, to, kDINeighbors);
+        poolTrace<kCount>(S, st, pool, count, ctr);
+        if (check && (pool.blocked[lane] >> kDINeighbors) & 1u) resv.resampleWeight = 0.0f;
+    }
+    if (inside) diShade(S, cam, px, resv, thisR, p, directOut, surface);
 }
 
 __global__ void k_di_reset(DIPlanes R) {
@@ -427,9 +535,14 @@ hipError_t launchDiTemporal(const rt_device_scene* s, const rt_camera* cams, con
 hipError_t launchDiSpatial(const rt_device_scene* s, const rt_camera* cams, const rt_frame& f,
                            const rt_di_reservoirs& r, const rt_di_settings& set, hipStream_t stream) {
     GB g = makeGB(f.depthNormal, f.albedoMatId, f.motionVector, f.width, f.height);
-    RT_DI_DISPATCH(k_di_spatial, set.shiftType, tileGrid(f.width, f.height), stream, s->dev, cams[0], g, set,
-                   diPlanes(r.reservoirTemp, f.width, f.height), diPlanes(r.reservoir, f.width, f.height),
-                   f.directOutput);
+    const DIPlanes tempR = diPlanes(r.reservoirTemp, f.width, f.height), thisR = diPlanes(r.reservoir, f.width, f.height);
+    TraceCounters* ctr = gCountersEnabled ? counterBuffer() : nullptr;
+    const auto kernel = set.shiftType == kShiftReconnection ? (gCountersEnabled ? k_di_spatial_pool<true> : k_di_spatial_pool<false>)
+                        : set.shiftType == kShiftReplay
+                            ? (gCountersEnabled ? k_di_spatial<true, kShiftReplay> : k_di_spatial<false, kShiftReplay>)
+                            : (gCountersEnabled ? k_di_spatial<true, 2u> : k_di_spatial<false, 2u>);
+    (void)launch(kernel, tileGrid(f.width, f.height), kTileThreads, stream, s->dev, cams[0], g, set, tempR, thisR,
+                 f.directOutput, ctr);
     return hipGetLastError();
 }
 

@@ -100,23 +100,86 @@ RT_DEV bool unpackGB(f4 dn, uint2 am, GPix& p) {
 template <bool kCount, bool kCull = true>
 RT_DEV Isec traceClosestHit(const DevScene& S, TStack st, f3 o, float tmin, f3 d, float tmax, TraceCounters* ctr,
                             bool skipLights = false, float* tOut = nullptr) {
-    RayT r = makeRay(o, d, tmin, tmax);
     Isec h; h.b1 = 0.0f; h.b2 = 0.0f; h.inst = RT_INVALID_HIT; h.prim = 0;
     float tBest = tmax;
-    bool hit = traverse<false, kCount, kCull>(S, r, skipLights, st, tBest, h, ctr);
+    bool hit = traverse<false, kCount, kCull>(S, o, d, tmin, skipLights, st, tBest, h, ctr);
     if (!hit) { h.inst = RT_INVALID_HIT; h.b1 = 0.0f; h.b2 = 0.0f; h.prim = 0; }
     if (tOut) *tOut = hit ? tBest : 0.0f;
     return h;
 }
 template <bool kCount>
 RT_DEV bool traceShadow(const DevScene& S, TStack st, f3 o, float tmin, f3 d, float tmax, TraceCounters* ctr) {
-    RayT r = makeRay(o, d, tmin, tmax);
     Isec h; float tBest = tmax;
-    return traverse<true, kCount>(S, r, false, st, tBest, h, ctr);
+    return traverse<true, kCount>(S, o, d, tmin, false, st, tBest, h, ctr);
 }
 template <bool kCount>
 RT_DEV bool traceVisibility(const DevScene& S, TStack st, f3 from, f3 to, TraceCounters* ctr) {
     return !traceShadow<kCount>(S, st, from, RT_MIN_RAY, normalize(to - from), distance(to, from) - RT_MIN_RAY, ctr);
+}
+
+// A wave's visibility rays, gathered in LDS so that its lanes can trace them without waiting for each other:
+// ray k runs from the origin of lane owner[k] & 63 to target[k]; an occluded one sets bit owner[k] >> 6 of that
+// lane's `blocked` word.
+template <uint32_t kRays>
+struct VisibilityPool {
+    float origin[3][kTileThreads];
+    float target[3][kRays];
+    uint32_t blocked[kTileThreads];
+    uint16_t owner[kRays];
+};
+// Lanes refilled at once (a new ray's set-up is issued for all of a refill's lanes).
+constexpr int kPoolRefill = 16;
+constexpr int kPoolStackWords = 16;  // LDS stack entries of a lane (any-hit rays keep one word each)
+
+// Appends this lane's ray (where want) to the pool; `count` is the wave's ray count. The wave is converged.
+template <uint32_t kRays>
+RT_DEV void poolAdd(VisibilityPool<kRays>& pool, uint32_t& count, bool want, f3 to, uint32_t bit) {
+    const unsigned long long mask = __ballot(want);
+    if (want) {
+        const uint32_t k = count + (uint32_t)__popcll(mask & ((1ull << threadIdx.x) - 1ull));
+        pool.target[0][k] = to.x; pool.target[1][k] = to.y; pool.target[2][k] = to.z;
+        pool.owner[k] = (uint16_t)(threadIdx.x | bit << 6);
+    }
+    count += (uint32_t)__popcll(mask);
+}
+
+// Traces the pool's `count` rays (traceVisibility of each) and empties it. All 64 lanes of the one-wave
+// workgroup call it.
+template <bool kCount, uint32_t kRays>
+RT_DEV void poolTrace(const DevScene& S, TStack st, VisibilityPool<kRays>& pool, uint32_t& count, TraceCounters* ctr) {
+    __syncthreads();
+    StackSpill spill;
+    WalkWork work{0, 0};
+    unsigned long long rays = 0;
+    Walk w;
+    w.cur = RT_EMPTY;
+    Isec h;
+    h.inst = RT_EMPTY;
+    uint32_t next = 0, owner = 0;
+    for (;;) {
+        if (w.cur == RT_EMPTY && h.inst != RT_EMPTY) {
+            atomicOr(&pool.blocked[owner & 63u], 1u << (owner >> 6));
+            h.inst = RT_EMPTY;
+        }
+        const unsigned long long idle = __ballot(w.cur == RT_EMPTY);
+        if (next >= count && idle == ~0ull) break;
+        if (w.cur == RT_EMPTY) {
+            const uint32_t k = next + (uint32_t)__popcll(idle & ((1ull << threadIdx.x) - 1ull));
+            if (k < count) {
+                owner = pool.owner[k];
+                const uint32_t l = owner & 63u;
+                const f3 from = mk3(pool.origin[0][l], pool.origin[1][l], pool.origin[2][l]);
+                const f3 to = mk3(pool.target[0][k], pool.target[1][k], pool.target[2][k]);
+                startWalk(S, w, from, normalize(to - from), RT_MIN_RAY, distance(to, from) - RT_MIN_RAY);
+                if (kCount) rays++;
+            }
+        }
+        next = min(count, next + (uint32_t)__popcll(idle));
+        walk<true, kCount, false, kPoolStackWords>(S, w, false, st, spill, next < count ? kTileThreads - kPoolRefill + 1 : 1, h, work);
+    }
+    if (kCount) countWork(ctr, work, rays);
+    count = 0;
+    __syncthreads();
 }
 
 RT_DEV void accumulate(float* out, size_t p, f3 c, uint32_t frameIndex) {

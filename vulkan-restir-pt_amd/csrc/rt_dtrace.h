@@ -45,6 +45,7 @@
 #define RT_LDS_STACK 11
 #endif
 #define RT_SPILL_STACK 244
+#define RT_MAX_STACK (RT_LDS_STACK + RT_SPILL_STACK)
 // Leaf tests are issued once RT_LEAF_SHARE x the lanes holding a leaf reach the lanes at a node.
 #ifndef RT_LEAF_SHARE
 #define RT_LEAF_SHARE 2
@@ -133,7 +134,7 @@ RT_DEV bool triHit(const RayT& r, f3 v0, f3 v1, f3 v2, float tBest, float& tOut,
         W = (float)((double)Bx * (double)Ay - (double)By * (double)Ax);
     }
     // one sign throughout, else the ray passes outside; no branches, so a wave's lanes leave together
-    const bool inside = (fminf(fminf(U, V), W) >= 0.0f) | (fmaxf(fmaxf(U, V), W) <= 0.0f);
+    const bool inside = fminf(fminf(U, V), W) >= 0.0f || fmaxf(fmaxf(U, V), W) <= 0.0f;
     float det = U + V + W;
     float Az = r.Sz * Akz, Bz = r.Sz * Bkz, Cz = r.Sz * Ckz;
     float T = U * Az + V * Bz + W * Cz;
@@ -153,15 +154,15 @@ struct TStack {
     uint32_t stride;
 };
 
-// The LDS of a block's traversal stacks: RT_LDS_STACK entries of two words per lane (a child
+// The LDS of a block's traversal stacks, kWords words per lane: RT_LDS_STACK entries of two words (a child
 // reference and its key), or twice as many of one word where no keys are kept.
-template <int kThreads>
+template <int kThreads, int kWords = 2 * RT_LDS_STACK>
 struct StackLDS {
-    uint32_t word[2 * RT_LDS_STACK * kThreads];
+    uint32_t word[kWords * kThreads];
 };
 
-template <int kThreads>
-RT_DEV TStack laneStack(StackLDS<kThreads>& s) {
+template <int kThreads, int kWords>
+RT_DEV TStack laneStack(StackLDS<kThreads, kWords>& s) {
     return TStack{(LdsWord*)s.word + threadIdx.x, (uint32_t)kThreads};
 }
 
@@ -182,27 +183,47 @@ RT_DEV void order2(int& ka, uint32_t& ra, int& kb, uint32_t& rb) {
     ra = t;
 }
 
-// kCull: closest-hit queries drop popped nodes beyond the closest hit (the
-// result is the same either way; the reuse passes' replays, which rarely pop
-// such nodes, leave it off to save registers).
-template <bool kAny, bool kCount, bool kCull = true>
-RT_DEV bool traverse(const DevScene& S, const RayT& r, bool skipLights, TStack st, float& tBest, Isec& hit,
-                     TraceCounters* ctr) {
-    constexpr bool kKeep = kCull && !kAny;  // keys kept on the stack
-    constexpr int kWords = kKeep ? 2 : 1;
-    constexpr int kCap = 2 * RT_LDS_STACK / kWords;
-    uint32_t spill[RT_SPILL_STACK];
-    uint16_t spillKey[kKeep ? RT_SPILL_STACK : 1];
-    const int entry = kWords * (int)st.stride;
-    int sp = 0;
-    unsigned long long cn = 0, ct = 0;
-    hit.inst = RT_EMPTY;
-    if (S.numPrims == 0) return false;
+// One lane's ray under way: idle when cur is RT_EMPTY, else at node or leaf cur with sp stack entries.
+struct Walk {
+    RayT r;
+    float tBest;
+    uint32_t cur;
+    int sp;
+};
+// The part of a lane's stack beyond its LDS entries (it must outlive the calls of walk() that a ray takes).
+struct StackSpill {
+    uint32_t ref[RT_SPILL_STACK];
+    uint16_t key[RT_SPILL_STACK];
+};
+struct WalkWork { unsigned long long nodes, tris; };
+
+RT_DEV void startWalk(const DevScene& S, Walk& w, f3 o, f3 d, float tmin, float tmax) {
+    w.r = makeRay(o, d, tmin, tmax);
+    w.tBest = tmax;
+    w.sp = 0;
     // A non-finite ray hits nothing; reject it here, because the slab test
     // (fminf/fmaxf drop NaN operands) would accept every box and the ray would
     // walk the whole tree.
-    uint32_t cur = isfinite(r.o.x) && isfinite(r.o.y) && isfinite(r.o.z) && isfinite(r.d.x) && isfinite(r.d.y) &&
-                           isfinite(r.d.z) ? 0u : RT_EMPTY;
+    w.cur = isfinite(o.x) && isfinite(o.y) && isfinite(o.z) && isfinite(d.x) && isfinite(d.y) && isfinite(d.z) &&
+                    S.numPrims != 0u ? 0u : RT_EMPTY;
+}
+
+// Walks the lanes' rays until fewer than minBusy of the wave's (converged) lanes are busy. kAny: a lane stops at
+// its first hit. hit.inst is set on a hit and is the caller's to initialise. kCull: closest-hit queries drop
+// popped nodes beyond the closest hit (the result is the same either way; the reuse passes' replays, which rarely
+// pop such nodes, leave it off to save registers).
+template <bool kAny, bool kCount, bool kCull, int kStackWords = 2 * RT_LDS_STACK>
+RT_DEV void walk(const DevScene& S, Walk& w, bool skipLights, TStack st, StackSpill& spill, int minBusy, Isec& hit,
+                 WalkWork& work) {
+    constexpr bool kKeep = kCull && !kAny;  // keys kept on the stack
+    constexpr int kWords = kKeep ? 2 : 1;
+    constexpr int kCap = kStackWords / kWords;
+    static_assert(kCap + RT_SPILL_STACK >= RT_MAX_STACK, "the build bounds the stack depth by RT_MAX_STACK");
+    const int entry = kWords * (int)st.stride;
+    const RayT& r = w.r;
+    float tBest = w.tBest;
+    uint32_t cur = w.cur;
+    int sp = w.sp;
     auto popOne = [&]() {
         sp--;
         uint32_t ref;
@@ -212,8 +233,8 @@ RT_DEV bool traverse(const DevScene& S, const RayT& r, bool skipLights, TStack s
             ref = e[0];
             if (kKeep) t = __uint_as_float(e[st.stride]);
         } else {
-            ref = spill[sp - kCap];
-            if (kKeep) t = __uint_as_float((uint32_t)spillKey[sp - kCap] << 16);
+            ref = spill.ref[sp - kCap];
+            if (kKeep) t = __uint_as_float((uint32_t)spill.key[sp - kCap] << 16);
         }
         if (kCount) t = __uint_as_float(__float_as_uint(t) & 0xffff0000u);
         cur = kKeep && t > tBest ? RT_EMPTY : ref;
@@ -226,15 +247,15 @@ RT_DEV bool traverse(const DevScene& S, const RayT& r, bool skipLights, TStack s
             popOne();
         }
     };
-    unsigned long long nodeLanes = __ballot((int)cur >= 0), leafLanes = 0;
-    while (nodeLanes | leafLanes) {
+    unsigned long long nodeLanes = __ballot((int)cur >= 0), leafLanes = __ballot((int)cur < -1);
+    while (__popcll(nodeLanes | leafLanes) >= minBusy) {
         if (RT_LEAF_SHARE * __popcll(leafLanes) >= __popcll(nodeLanes)) {
             if ((int)cur < -1) {
                 const float4* tp = S.leafTris + 3 * (size_t)(cur & ~RT_LEAF);
                 const float4 a = tp[0], b = tp[1], c = tp[2];
                 const uint32_t inst = __float_as_uint(a.w);
                 const bool skip = skipLights & (inst == 0u);
-                if (kCount) ct += skip ? 0 : 1;
+                if (kCount) work.tris += skip ? 0 : 1;
                 float t, b1, b2;
                 const bool h = triHit(r, mk3(a.x, a.y, a.z), mk3(b.x, b.y, b.z), mk3(c.x, c.y, c.z), tBest, t, b1, b2);
                 cur = RT_EMPTY;
@@ -256,7 +277,7 @@ RT_DEV bool traverse(const DevScene& S, const RayT& r, bool skipLights, TStack s
             const float4 ny = *reinterpret_cast<const float4*>(np + r.ny), fy = *reinterpret_cast<const float4*>(np + (r.ny ^ 80u));
             const float4 nz = *reinterpret_cast<const float4*>(np + r.nz), fz = *reinterpret_cast<const float4*>(np + (r.nz ^ 112u));
             const float4 cr = *reinterpret_cast<const float4*>(np + 96);
-            if (kCount) cn++;
+            if (kCount) work.nodes++;
             uint32_t c0 = __float_as_uint(cr.x), c1 = __float_as_uint(cr.y), c2 = __float_as_uint(cr.z),
                      c3 = __float_as_uint(cr.w);
             float t0, t1, t2, t3;
@@ -302,8 +323,8 @@ RT_DEV bool traverse(const DevScene& S, const RayT& r, bool skipLights, TStack s
                         st.lds[pos * entry] = cs[q];
                         if (kKeep) st.lds[pos * entry + (int)st.stride] = key[q];
                     } else if (pos - kCap < RT_SPILL_STACK) {  // the build bounds the stack depth
-                        spill[pos - kCap] = cs[q];
-                        if (kKeep) spillKey[pos - kCap] = (uint16_t)(key[q] >> 16);
+                        spill.ref[pos - kCap] = cs[q];
+                        if (kKeep) spill.key[pos - kCap] = (uint16_t)(key[q] >> 16);
                     }
                 }
             }
@@ -314,7 +335,27 @@ RT_DEV bool traverse(const DevScene& S, const RayT& r, bool skipLights, TStack s
         nodeLanes = __ballot((int)cur >= 0);
         leafLanes = __ballot((int)cur < -1);
     }
-    if (kCount) { atomicAdd(&ctr->nodes, cn); atomicAdd(&ctr->tris, ct); atomicAdd(&ctr->rays, 1ull); }
+    w.tBest = tBest;
+    w.cur = cur;
+    w.sp = sp;
+}
+
+RT_DEV void countWork(TraceCounters* ctr, const WalkWork& work, unsigned long long rays) {
+    atomicAdd(&ctr->nodes, work.nodes); atomicAdd(&ctr->tris, work.tris); atomicAdd(&ctr->rays, rays);
+}
+
+// One ray per lane, to the end.
+template <bool kAny, bool kCount, bool kCull = true>
+RT_DEV bool traverse(const DevScene& S, f3 o, f3 d, float tmin, bool skipLights, TStack st, float& tBest, Isec& hit,
+                     TraceCounters* ctr) {
+    StackSpill spill;
+    WalkWork work{0, 0};
+    Walk w;
+    startWalk(S, w, o, d, tmin, tBest);
+    hit.inst = RT_EMPTY;
+    walk<kAny, kCount, kCull>(S, w, skipLights, st, spill, 1, hit, work);
+    tBest = w.tBest;
+    if (kCount && S.numPrims != 0u) countWork(ctr, work, 1ull);
     return hit.inst != RT_EMPTY;
 }
 
