@@ -67,6 +67,7 @@ struct rt_mlp {
     float* wM = nullptr;
     float* wV = nullptr;
     float* partial = nullptr;     // per-wave weight-gradient partial sums
+    float2* encGrad = nullptr;    // encoding gradients of a batch of up to kBatchCap samples: [level][sample]
     uint32_t partialWaves = 0;
     float* batchPos = nullptr;    // training batch gathered from the frame
     float* batchTarget = nullptr;

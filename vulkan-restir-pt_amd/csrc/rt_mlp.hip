@@ -201,11 +201,15 @@ __device__ __forceinline__ void vmfLoss(const Fwd& F, int h, const float wd[3], 
 // Targets: 3 floats per sample (radiance network: RGB, negative = masked) or 4 (proposal
 // network: unit direction and weight; weight <= 0 or non-finite = masked). wmean: the mean
 // weight of the valid samples (proposal network only).
-template <int kO>
+//
+// kStore: the encoding gradients go to encGrad[level][sample] for k_mlp_scatter; otherwise (batches beyond
+// kBatchCap samples) they are added to the table here.
+template <int kO, bool kStore>
 __global__ __launch_bounds__(64) void k_mlp_train(MlpView M, const float* __restrict__ pos,
                                                   const float* __restrict__ target, uint32_t n,
                                                   const float* __restrict__ wmean,
-                                                  long long* __restrict__ gridGrad, float* __restrict__ partial) {
+                                                  long long* __restrict__ gridGrad, float2* __restrict__ encGrad,
+                                                  float* __restrict__ partial) {
     constexpr int kSteps = (kO + 7) / 8;  // k-steps over the outputs
     constexpr int kTS = kO == kOut ? 3 : 4;  // target stride
     __shared__ TrainLDS<kO> L;
@@ -281,8 +285,14 @@ __global__ __launch_bounds__(64) void k_mlp_train(MlpView M, const float* __rest
             denc = mfma2(bwdA(L.w + kW1, kHidden, j, 8 * s8 + 4 * h, kHidden), b0,
                          bwdA(L.w + kW1, kHidden, j, 8 * (s8 + 1) + 4 * h, kHidden), b1, denc);
         }
-        // scatter the encoding gradient: register group g holds levels 4g + 2h (+1)
-        if (s < n && valid) {
+        // the encoding gradient: register group g holds levels 4g + 2h (+1)
+        if constexpr (kStore) {
+            if (s < n)
+                for (int g = 0; g < 4; g++)
+                    for (int q = 0; q < 2; q++)
+                        encGrad[(size_t)(4 * g + 2 * h + q) * kBatchCap + s] =
+                            valid ? make_float2(denc[4 * g + 2 * q], denc[4 * g + 2 * q + 1]) : make_float2(0.0f, 0.0f);
+        } else if (s < n && valid) {
             for (int g = 0; g < 4; g++) {
                 for (int q = 0; q < 2; q++) {
                     const int lev = 4 * g + 2 * h + q;
@@ -366,6 +376,41 @@ __global__ __launch_bounds__(64) void k_mlp_train(MlpView M, const float* __rest
         count += __shfl_xor(count, off);
     }
     if (lane == 0) { P[weightsFor(kO)] = lossSum; P[weightsFor(kO) + 1] = count; }
+}
+
+// Adds a batch's encoding gradients to the grid-gradient table (32.32 fixed point: the sums do not depend on
+// the order). What bounds it is the atomics: each sample adds to 8 corners x 2 features of 16 levels. Added from all
+// over the GPU, a table line moves between the 8 XCDs' L2s with every few adds; so level l is added by the
+// workgroups of one XCD only (workgroups are dealt to the XCDs round robin), XCD x taking levels x and 15 - x, a
+// coarse level, whose few corners all samples share, with a fine one. Four lanes take a sample's two features at
+// two corners neighbouring in x, which are adjacent in a dense table and, for an even x, in a hashed one.
+constexpr uint32_t kXcds = 8;
+constexpr uint32_t kScatterThreads = 256, kScatterBlocks = 128;  // per XCD
+__global__ __launch_bounds__(kScatterThreads) void k_mlp_scatter(MlpView M, const float* __restrict__ pos, uint32_t n,
+                                                                 const float2* __restrict__ encGrad,
+                                                                 long long* __restrict__ gridGrad) {
+    const uint32_t xcd = blockIdx.x % kXcds, part = blockIdx.x / kXcds;
+    const uint32_t f = threadIdx.x & 1u, xbit = (threadIdx.x >> 1) & 1u;
+    constexpr uint32_t kSamples = kScatterThreads / 4;
+    for (int pass = 0; pass < 2; pass++) {
+        const int lev = pass == 0 ? kLevels - 1 - (int)xcd : (int)xcd;
+        const float* d = reinterpret_cast<const float*>(encGrad + (size_t)lev * kBatchCap);
+        for (uint32_t s = part * kSamples + (threadIdx.x >> 2); s < n; s += kScatterBlocks * kSamples) {
+            const float g = d[2 * (size_t)s + f];
+            float u, v, w;
+            normalizePos(M, pos[3 * (size_t)s], pos[3 * (size_t)s + 1], pos[3 * (size_t)s + 2], u, v, w);
+            uint32_t ci[3]; float fr[3];
+            levelCell(M, lev, u, v, w, ci, fr);
+#pragma unroll
+            for (int yz = 0; yz < 4; yz++) {
+                const Corner k = corner(M, lev, ci, fr, (int)xbit + 2 * yz);
+                const long long a = __float2ll_rn(k.wt * g * kFix);
+                if (a != 0)
+                    atomicAdd(reinterpret_cast<unsigned long long*>(gridGrad + 2 * (size_t)k.slot) + f,
+                              (unsigned long long)a);
+            }
+        }
+    }
 }
 
 // Mean weight of the valid samples of a proposal batch (one workgroup, fixed-order sums).
@@ -461,7 +506,7 @@ rt_status invalid(const char* m) { rti::setError(m); return RT_ERR_INVALID_ARGUM
 void freeMlp(rt_mlp* m) {
     (void)hipFree(m->gridF32); (void)hipFree(m->gridF16); (void)hipFree(m->gridGrad); (void)hipFree(m->gridM);
     (void)hipFree(m->gridV); (void)hipFree(m->wF32); (void)hipFree(m->wF16); (void)hipFree(m->wGrad);
-    (void)hipFree(m->wM); (void)hipFree(m->wV); (void)hipFree(m->partial); (void)hipFree(m->batchPos);
+    (void)hipFree(m->wM); (void)hipFree(m->wV); (void)hipFree(m->partial); (void)hipFree(m->encGrad); (void)hipFree(m->batchPos);
     (void)hipFree(m->batchTarget); (void)hipFree(m->wmean);
     delete m;
 }
@@ -486,16 +531,20 @@ hipError_t mlpGradients(rt_mlp* m, const float* pos, const float* target, uint32
     (void)launch(k_fill_i64, dim3(blocks(m->gridParams, 256)), dim3(256), st, m->gridGrad, m->gridParams);
     const uint32_t tiles = (n + kTileSamples - 1) / kTileSamples;
     const uint32_t waves = std::max(1u, std::min(tiles, m->partialWaves));
+    const bool store = n <= kBatchCap;
     if (n && guide) {
         (void)launch(k_guide_wmean, dim3(1), dim3(kMeanThreads), st, target, n, m->wmean);
-        (void)launch(k_mlp_train<kGuideOut>, dim3(waves), dim3(64), st, m->view, pos, target, n, (const float*)m->wmean,
-                     m->gridGrad, m->partial);
+        (void)launch(store ? k_mlp_train<kGuideOut, true> : k_mlp_train<kGuideOut, false>, dim3(waves), dim3(64), st, m->view,
+                     pos, target, n, (const float*)m->wmean, m->gridGrad, m->encGrad, m->partial);
     } else if (n) {
-        (void)launch(k_mlp_train<kOut>, dim3(waves), dim3(64), st, m->view, pos, target, n, (const float*)nullptr,
-                     m->gridGrad, m->partial);
+        (void)launch(store ? k_mlp_train<kOut, true> : k_mlp_train<kOut, false>, dim3(waves), dim3(64), st, m->view, pos,
+                     target, n, (const float*)nullptr, m->gridGrad, m->encGrad, m->partial);
     } else {
         (void)launch(k_fill_f32, dim3(blocks(stride, 256)), dim3(256), st, m->partial, (uint64_t)stride, 0.0f);
     }
+    if (n && store)
+        (void)launch(k_mlp_scatter, dim3(kXcds * kScatterBlocks), dim3(kScatterThreads), st, m->view, pos, n,
+                     (const float2*)m->encGrad, m->gridGrad);
     const uint32_t rows = n ? waves : 1u;
     const uint32_t groups = (rows + kReduceGroup - 1u) / kReduceGroup;
     (void)launch(k_mlp_reduce_groups, dim3(blocks(stride, 256), groups), dim3(256), st, m->partial, rows, stride);
@@ -570,6 +619,7 @@ rt_status createNet(const rt_mlp_config* c, uint32_t outputs, hipStream_t stream
               rti::hipCheck(hipMalloc(&m->wM, 4 * NW), "hipMalloc") &&
               rti::hipCheck(hipMalloc(&m->wV, 4 * NW), "hipMalloc") &&
               rti::hipCheck(hipMalloc(&m->partial, 4 * (size_t)stride * kMaxTrainWaves), "hipMalloc") &&
+              rti::hipCheck(hipMalloc(&m->encGrad, sizeof(float2) * kLevels * kBatchCap), "hipMalloc") &&
               rti::hipCheck(hipMalloc(&m->batchPos, sizeof(float) * 3 * kBatchCap), "hipMalloc") &&
               rti::hipCheck(hipMalloc(&m->batchTarget, sizeof(float) * m->targetStride * kBatchCap), "hipMalloc") &&
               rti::hipCheck(hipMalloc(&m->wmean, sizeof(float)), "hipMalloc");
