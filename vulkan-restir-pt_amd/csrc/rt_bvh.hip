@@ -6,7 +6,7 @@
 //   2. centroid bounds: per-block min/max then one final block
 //   3. 63-bit Morton codes of quantised centroids
 //   4. stable LSD radix sort of (code, primitive) pairs: 8 passes of 8-bit
-//      digits; per block a 256-bin histogram, one exclusive scan over
+//      digits, in one workgroup up to 4096 pairs; beyond, per block a 256-bin histogram, one exclusive scan over
 //      (digit, block), then a scatter whose in-block rank comes from 8 wave
 //      ballots (equal-digit lane masks) plus per-wave digit counts in LDS
 //   5. Karras topology, one thread per internal node
@@ -25,7 +25,6 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr int kItems = 16;
-constexpr int kTile = kBlock * kItems;
 constexpr uint32_t kNoParent = 0xffffffffu;
 
 __device__ __forceinline__ uint64_t expandBits21(uint64_t v) {
@@ -166,17 +165,31 @@ __device__ __forceinline__ uint32_t blockExclusiveScan(uint32_t v, uint32_t* tot
     return base + inc - v;
 }
 
-// 4. radix sort
+// 4. radix sort, in tiles of 256 kI keys. A workgroup goes through its tile in kI rounds of barriers, so a sort of few
+// keys is faster over many small tiles: at 100k keys a pass's scatter takes 16.5 us with kI = 16 (25 workgroups), 5.4
+// with kI = 2, the whole build 354 -> 188 us.
+constexpr uint32_t kSmallSort = 4096;  // up to which one workgroup sorts in LDS (k_radix_sort_small)
+inline int radixItems(uint32_t n) { return n <= (1u << 18) ? 2 : (n <= (1u << 20) ? 4 : 16); }
+inline uint32_t radixTiles(uint32_t n) {
+    const uint32_t tile = (uint32_t)kBlock * (uint32_t)radixItems(n);
+    return n / tile + (n % tile ? 1u : 0u);
+}
+template <int kI>
 __global__ void k_radix_hist(const unsigned long long* __restrict__ keys, uint32_t n, int shift, uint32_t nBlocks,
                              uint32_t* __restrict__ blockHist) {
     __shared__ uint32_t h[256];
     h[threadIdx.x] = 0;
     __syncthreads();
-    uint32_t base = blockIdx.x * kTile;
-    for (int k = 0; k < kItems; k++) {
-        uint32_t i = base + k * kBlock + threadIdx.x;
-        if (i < n) atomicAdd(&h[(uint32_t)(keys[i] >> shift) & 0xffu], 1u);
+    uint32_t base = blockIdx.x * (kBlock * kI);
+    unsigned long long key[kI];
+#pragma unroll
+    for (int k = 0; k < kI; k++) {
+        const uint32_t i = base + k * kBlock + threadIdx.x;
+        key[k] = i < n ? keys[i] : 0ull;
     }
+#pragma unroll
+    for (int k = 0; k < kI; k++)
+        if (base + k * kBlock + threadIdx.x < n) atomicAdd(&h[(uint32_t)(key[k] >> shift) & 0xffu], 1u);
     __syncthreads();
     blockHist[threadIdx.x * nBlocks + blockIdx.x] = h[threadIdx.x];
 }
@@ -201,6 +214,7 @@ __global__ void k_radix_digit_scan(uint32_t* __restrict__ blockHist, uint32_t nB
 // (scan of the digit totals), plus the count of its digit in earlier blocks,
 // plus its rank among equal digits earlier in the block (8 wave ballots give
 // the equal-digit lane mask; per-wave digit counts go through LDS).
+template <int kI>
 __global__ void k_radix_scatter(const unsigned long long* __restrict__ keysIn, const uint32_t* __restrict__ valsIn,
                                 uint32_t n, int shift, uint32_t nBlocks, const uint32_t* __restrict__ blockOffset,
                                 const uint32_t* __restrict__ digitTotal, unsigned long long* __restrict__ keysOut,
@@ -214,12 +228,21 @@ __global__ void k_radix_scatter(const unsigned long long* __restrict__ keysIn, c
     for (int w = 0; w < kBlock / 64; w++) waveCnt[w][tid] = 0;
     __syncthreads();
     const unsigned long long ltMask = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
-    uint32_t base = blockIdx.x * kTile;
-    for (int k = 0; k < kItems; k++) {
+    uint32_t base = blockIdx.x * (kBlock * kI);
+    unsigned long long keys[kI];
+    uint32_t vals[kI];
+#pragma unroll
+    for (int k = 0; k < kI; k++) {
+        const uint32_t i = base + k * kBlock + tid;
+        keys[k] = i < n ? keysIn[i] : 0ull;
+        vals[k] = i < n ? valsIn[i] : 0u;
+    }
+#pragma unroll
+    for (int k = 0; k < kI; k++) {
         uint32_t i = base + k * kBlock + tid;
         bool valid = i < n;
-        unsigned long long key = valid ? keysIn[i] : 0ull;
-        uint32_t val = valid ? valsIn[i] : 0u;
+        const unsigned long long key = keys[k];
+        const uint32_t val = vals[k];
         uint32_t d = (uint32_t)(key >> shift) & 0xffu;
         unsigned long long mask = __ballot(valid);
         for (int b = 0; b < 8; b++) {
@@ -241,6 +264,82 @@ __global__ void k_radix_scatter(const unsigned long long* __restrict__ keysIn, c
         for (int w = 0; w < kBlock / 64; w++) { tot += waveCnt[w][tid]; waveCnt[w][tid] = 0; }
         running[tid] += tot;
         __syncthreads();
+    }
+}
+
+// The whole sort of up to kSmallSort keys in one workgroup: the same stable passes with the pairs in LDS, instead of
+// 24 launches of a few microseconds each. Thread t holds the pairs at t, t + 1024, ... of the current order.
+constexpr uint32_t kSmallThreads = 1024, kSmallItems = kSmallSort / kSmallThreads;
+__global__ __launch_bounds__(kSmallThreads) void k_radix_sort_small(unsigned long long* __restrict__ keys,
+                                                                   uint32_t* __restrict__ vals, uint32_t n) {
+    __shared__ unsigned long long sk[kSmallSort];
+    __shared__ uint32_t sv[kSmallSort];
+    __shared__ uint32_t running[256];
+    __shared__ uint16_t waveCnt[kSmallThreads / 64][256];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    const unsigned long long ltMask = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
+    const uint32_t rounds = (n + kSmallThreads - 1u) / kSmallThreads;
+    unsigned long long key[kSmallItems];
+    uint32_t val[kSmallItems];
+#pragma unroll
+    for (uint32_t k = 0; k < kSmallItems; k++) {
+        const uint32_t i = k * kSmallThreads + tid;
+        key[k] = i < n ? keys[i] : 0ull;
+        val[k] = i < n ? vals[i] : 0u;
+    }
+    for (uint32_t w = 0; w < kSmallThreads / 64; w++)
+        if (tid < 256u) waveCnt[w][tid] = 0;
+    for (int pass = 0; pass < 8; pass++) {
+        const int shift = pass * 8;
+        if (tid < 256u) running[tid] = 0u;
+        __syncthreads();
+#pragma unroll
+        for (uint32_t k = 0; k < kSmallItems; k++)
+            if (k * kSmallThreads + tid < n) atomicAdd(&running[(uint32_t)(key[k] >> shift) & 0xffu], 1u);
+        __syncthreads();
+        const uint32_t count = tid < 256u ? running[tid] : 0u;
+        uint32_t total;
+        const uint32_t first = blockExclusiveScan(count, &total);
+        if (tid < 256u) running[tid] = first;
+        __syncthreads();
+#pragma unroll
+        for (uint32_t k = 0; k < kSmallItems; k++) {
+            if (k >= rounds) break;
+            const bool valid = k * kSmallThreads + tid < n;
+            const uint32_t d = (uint32_t)(key[k] >> shift) & 0xffu;
+            unsigned long long mask = __ballot(valid);
+            for (int b = 0; b < 8; b++) {
+                const bool bit = (d >> b) & 1u;
+                const unsigned long long bal = __ballot(bit);
+                mask &= bit ? bal : ~bal;
+            }
+            const uint32_t rank = (uint32_t)__popcll(mask & ltMask);
+            if (valid && rank == 0) waveCnt[wave][d] = (uint16_t)__popcll(mask);
+            __syncthreads();
+            if (valid) {
+                uint32_t off = running[d] + rank;
+                for (uint32_t w = 0; w < wave; w++) off += waveCnt[w][d];
+                sk[off] = key[k];
+                sv[off] = val[k];
+            }
+            __syncthreads();
+            if (tid < 256u) {
+                uint32_t tot = 0;
+                for (uint32_t w = 0; w < kSmallThreads / 64; w++) { tot += waveCnt[w][tid]; waveCnt[w][tid] = 0; }
+                running[tid] += tot;
+            }
+            __syncthreads();
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < kSmallItems; k++) {
+            const uint32_t i = k * kSmallThreads + tid;
+            if (i < n) { key[k] = sk[i]; val[k] = sv[i]; }
+        }
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < kSmallItems; k++) {
+        const uint32_t i = k * kSmallThreads + tid;
+        if (i < n) { keys[i] = key[k]; vals[i] = val[k]; }
     }
 }
 
@@ -368,17 +467,26 @@ __device__ __forceinline__ uint32_t mergeNode(const float* nf, const uint32_t* h
 // arrival is ordered by workgroup-scope fences only, which on this part need no
 // cache maintenance. A climb that reaches a node with leaves outside the
 // workgroup leaves its slot written and stops there (phase 2 takes over).
+//
+// A workgroup's time is its threads' climbs, one leaf after the other, each a chain of dependent fetches a level:
+// 1024 leaves a workgroup (one a thread) up to 512k primitives, 4096 beyond, where the top part, which one workgroup
+// finishes, would grow too long (100k primitives: 79 us over 25 workgroups of 4096 leaves, 23 over 98 of 1024; the
+// top part 47 -> 53 us).
 constexpr uint32_t kRefitThreads = 1024;
-constexpr uint32_t kRefitLeaves = 4096;
+constexpr uint32_t kRefitLeaves = 4096;  // at most, per workgroup
+inline int refitShift(uint32_t n) { return n <= (1u << 19) ? 10 : 12; }
+static_assert(kRefitLeaves == 1u << 12, "refitShift");
 
 __global__ __launch_bounds__(kRefitThreads) void k_refit_block(const float4* __restrict__ tris,
                                                                const uint32_t* __restrict__ order, uint32_t n,
                                                                float4* nodes, const uint32_t* __restrict__ parentI,
                                                                const uint32_t* __restrict__ parentL,
-                                                               const uint2* __restrict__ range, uint32_t* height) {
+                                                               const uint2* __restrict__ range, uint32_t* height,
+                                                               int shift) {
     __shared__ uint32_t arrivals[kRefitLeaves];
-    const uint32_t L0 = blockIdx.x * kRefitLeaves, L1 = min(n, L0 + kRefitLeaves);
-    for (uint32_t k = threadIdx.x; k < kRefitLeaves; k += kRefitThreads) arrivals[k] = 0u;
+    const uint32_t leaves = 1u << shift;
+    const uint32_t L0 = blockIdx.x << shift, L1 = min(n, L0 + leaves);
+    for (uint32_t k = threadIdx.x; k < leaves; k += kRefitThreads) arrivals[k] = 0u;
     __syncthreads();
     for (uint32_t i = L0 + threadIdx.x; i < L1; i += kRefitThreads) {
         const float4* t = tris + 3 * (size_t)(order ? order[i] : i);
@@ -418,10 +526,10 @@ constexpr uint32_t kMaxTopLevels = 128;
 
 __global__ __launch_bounds__(kRefitThreads) void k_refit_top(float4* nodes, const uint32_t* __restrict__ parentI,
                                                              const uint2* __restrict__ range, uint32_t n,
-                                                             uint32_t* height, uint32_t* list) {
+                                                             uint32_t* height, uint32_t* list, int shift) {
     __shared__ uint32_t levelEnd[kMaxTopLevels];
     __shared__ uint32_t tail, levels;
-    if (n <= kRefitLeaves) return;  // one block: phase 1 merged every node up to the root
+    if (n <= 1u << shift) return;  // one block: phase 1 merged every node up to the root
     if (threadIdx.x == 0) {
         list[0] = 0u;  // the root
         tail = 1u;
@@ -437,7 +545,7 @@ __global__ __launch_bounds__(kRefitThreads) void k_refit_top(float4* nodes, cons
                 const uint32_t c = __float_as_uint(nf[12 + k]);
                 if (c & RT_LEAF) continue;
                 const uint2 r = range[c];
-                if (r.x / kRefitLeaves != r.y / kRefitLeaves) list[atomicAdd(&tail, 1u)] = c;
+                if (r.x >> shift != r.y >> shift) list[atomicAdd(&tail, 1u)] = c;
             }
         }
         __syncthreads();
@@ -696,7 +804,7 @@ void scanExclusive(const uint32_t* in, uint32_t* out, uint32_t n, uint32_t* sums
 namespace rti {
 
 size_t carveLbvhScratch(uint32_t n, char* base, LbvhScratch* out) {
-    const size_t nTiles = cdiv(n, kTile), nb = std::min<uint32_t>(1024u, cdiv(n, kBlock));
+    const size_t nTiles = radixTiles(n), nb = std::min<uint32_t>(1024u, cdiv(n, kBlock));
     const size_t nNodes = n > 1 ? n - 1 : 1;
     size_t off = 0;
     auto take = [&](size_t bytes) {
@@ -728,21 +836,27 @@ size_t carveLbvhScratch(uint32_t n, char* base, LbvhScratch* out) {
 // scene's box lands in sc.box, the tree's height in sc.height[0].
 hipError_t launchBinaryBuild(const float4* primTris, uint32_t n, unsigned long long* codes, uint32_t* order,
                              float4* nodes, float4* leafTris, const LbvhScratch& sc, hipStream_t stream) {
-    const uint32_t nTiles = cdiv(n, kTile);
     const uint32_t nbBounds = std::min<uint32_t>(1024u, cdiv(n, kBlock));
     k_bounds_partial<<<nbBounds, kBlock, 0, stream>>>(primTris, n, sc.partial);
     k_bounds_final<<<1, kBlock, 0, stream>>>(sc.partial, nbBounds, sc.box);
     k_morton<<<cdiv(n, kBlock), kBlock, 0, stream>>>(primTris, n, sc.box, codes, order);
-    unsigned long long *kin = codes, *kout = sc.keysB;
-    uint32_t *vin = order, *vout = sc.valsB;
-    for (int pass = 0; pass < 8; pass++) {
-        const int shift = pass * 8;
-        k_radix_hist<<<nTiles, kBlock, 0, stream>>>(kin, n, shift, nTiles, sc.blockHist);
-        k_radix_digit_scan<<<256, kBlock, 0, stream>>>(sc.blockHist, nTiles, sc.digitTotal);
-        k_radix_scatter<<<nTiles, kBlock, 0, stream>>>(kin, vin, n, shift, nTiles, sc.blockHist, sc.digitTotal, kout,
-                                                       vout);
-        std::swap(kin, kout);
-        std::swap(vin, vout);
+    if (n <= kSmallSort) {
+        k_radix_sort_small<<<1, kSmallThreads, 0, stream>>>(codes, order, n);
+    } else {
+        const uint32_t nTiles = radixTiles(n);
+        const int items = radixItems(n);
+        const auto hist = items == 2 ? k_radix_hist<2> : (items == 4 ? k_radix_hist<4> : k_radix_hist<16>);
+        const auto scatter = items == 2 ? k_radix_scatter<2> : (items == 4 ? k_radix_scatter<4> : k_radix_scatter<16>);
+        unsigned long long *kin = codes, *kout = sc.keysB;
+        uint32_t *vin = order, *vout = sc.valsB;
+        for (int pass = 0; pass < 8; pass++) {
+            const int shift = pass * 8;
+            hist<<<nTiles, kBlock, 0, stream>>>(kin, n, shift, nTiles, sc.blockHist);
+            k_radix_digit_scan<<<256, kBlock, 0, stream>>>(sc.blockHist, nTiles, sc.digitTotal);
+            scatter<<<nTiles, kBlock, 0, stream>>>(kin, vin, n, shift, nTiles, sc.blockHist, sc.digitTotal, kout, vout);
+            std::swap(kin, kout);
+            std::swap(vin, vout);
+        }
     }
     // 8 passes: the sorted data is back in codes / order
     if (n == 1) {
@@ -758,9 +872,11 @@ hipError_t launchBinaryBuild(const float4* primTris, uint32_t n, unsigned long l
         tris = leafTris;
         refitOrder = nullptr;
     }
-    k_refit_block<<<cdiv(n, kRefitLeaves), kRefitThreads, 0, stream>>>(tris, refitOrder, n, nodes, sc.parentI,
-                                                                       sc.parentL, sc.range, sc.height);
-    k_refit_top<<<1, kRefitThreads, 0, stream>>>(nodes, sc.parentI, sc.range, n, sc.height, sc.topList);
+    const int shift = refitShift(n);
+    k_refit_block<<<cdiv(n, 1u << shift), kRefitThreads, 0, stream>>>(tris, refitOrder, n, nodes, sc.parentI,
+                                                                      sc.parentL, sc.range, sc.height, shift);
+    if (n > 1u << shift)
+        k_refit_top<<<1, kRefitThreads, 0, stream>>>(nodes, sc.parentI, sc.range, n, sc.height, sc.topList, shift);
     return hipGetLastError();
 }
 
