@@ -80,8 +80,10 @@ __device__ __forceinline__ void loadWeightsLDS(_Float16* sW, const _Float16* w) 
 
 // ---- inference ------------------------------------------------------------------------------
 // Radiance network: exp-activated RGB per sample. Proposal network: its 32 raw outputs per sample.
+// Held to four waves per SIMD (128 VGPRs): the gathers' latency bounds it (300k points: 172 us at the three waves of
+// its own allocation, 158 at four, 254 at five, where it spills).
 template <int kO>
-__global__ __launch_bounds__(64 * kInferWaves) void k_mlp_infer(MlpView M, const float* __restrict__ pos, uint32_t n,
+__global__ __launch_bounds__(64 * kInferWaves, 4) void k_mlp_infer(MlpView M, const float* __restrict__ pos, uint32_t n,
                                                                 float* __restrict__ out) {
     __shared__ _Float16 sW[weightsFor(kO)];
     loadWeightsLDS<kO>(sW, M.w);
@@ -238,7 +240,7 @@ __global__ __launch_bounds__(64) void k_mlp_train(MlpView M, const float* __rest
             valid = s < n && isfinite(y[3]) && y[3] > 0.0f && isfinite(y[0]) && isfinite(y[1]) && isfinite(y[2]) &&
                     invMean > 0.0f;
         h4 enc[4];
-        encodeLane(M, (uint32_t)h, u, v, w, enc);
+        encodeLane<false>(M, (uint32_t)h, u, v, w, enc);
         Fwd F;
         forwardTileT<kO>(L.w, lane, enc, F);
 
@@ -384,16 +386,57 @@ __global__ __launch_bounds__(64) void k_mlp_train(MlpView M, const float* __rest
 // workgroups of one XCD only (workgroups are dealt to the XCDs round robin), XCD x taking levels x and 15 - x, a
 // coarse level, whose few corners all samples share, with a fine one. Four lanes take a sample's two features at
 // two corners neighbouring in x, which are adjacent in a dense table and, for an even x, in a hashed one.
+// A level whose dense table fits in LDS has so few corners that even one XCD's adds wait for each other (168 of 287 us
+// for the coarse levels of 65536 points); k_mlp_scatter_lds sums those (9 us for two levels; the step 590 -> 532 us).
 constexpr uint32_t kXcds = 8;
+constexpr uint32_t kLdsEntries = 12288, kLdsParts = 16, kLdsThreads = 1024;
+// Workgroup (level, feature, part): the part's samples summed in an LDS table of the level's entries, then the
+// entries that are not zero added to the gradient table.
+__global__ __launch_bounds__(kLdsThreads) void k_mlp_scatter_lds(MlpView M, const float* __restrict__ pos, uint32_t n,
+                                                                 const float2* __restrict__ encGrad,
+                                                                 long long* __restrict__ gridGrad) {
+    __shared__ unsigned long long table[kLdsEntries];
+    const int lev = (int)(blockIdx.x / (2u * kLdsParts));
+    const uint32_t f = (blockIdx.x / kLdsParts) & 1u, part = blockIdx.x % kLdsParts;
+    const uint32_t r = M.res[lev] + 1u, entries = r * r * r, base = (uint32_t)lev * (M.tableMask + 1u);
+    for (uint32_t i = threadIdx.x; i < entries; i += kLdsThreads) table[i] = 0ull;
+    __syncthreads();
+    const float* d = reinterpret_cast<const float*>(encGrad + (size_t)lev * kBatchCap);
+    for (uint32_t s = part * kLdsThreads + threadIdx.x; s < n; s += kLdsParts * kLdsThreads) {
+        const float g = d[2 * (size_t)s + f];
+        float u, v, w;
+        normalizePos(M, pos[3 * (size_t)s], pos[3 * (size_t)s + 1], pos[3 * (size_t)s + 2], u, v, w);
+        uint32_t ci[3]; float fr[3];
+        levelCell(M, lev, u, v, w, ci, fr);
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
+            const Corner k = corner(M, lev, ci, fr, c);
+            const long long a = __float2ll_rn(k.wt * g * kFix);
+            if (a != 0) atomicAdd(&table[k.slot - base], (unsigned long long)a);
+        }
+    }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < entries; i += kLdsThreads)
+        if (table[i] != 0ull)
+            atomicAdd(reinterpret_cast<unsigned long long*>(gridGrad + 2 * ((size_t)base + i)) + f, table[i]);
+}
+// Levels [0, this) are dense with at most kLdsEntries entries (the resolution does not fall with the level).
+inline int ldsLevels(const MlpView& M) {
+    int l = 0;
+    while (l < kLevels && ((M.denseMask >> l) & 1u) && (uint64_t)(M.res[l] + 1u) * (M.res[l] + 1u) * (M.res[l] + 1u) <= kLdsEntries) l++;
+    return l;
+}
+
 constexpr uint32_t kScatterThreads = 256, kScatterBlocks = 128;  // per XCD
 __global__ __launch_bounds__(kScatterThreads) void k_mlp_scatter(MlpView M, const float* __restrict__ pos, uint32_t n,
-                                                                 const float2* __restrict__ encGrad,
+                                                                 const float2* __restrict__ encGrad, int firstLevel,
                                                                  long long* __restrict__ gridGrad) {
     const uint32_t xcd = blockIdx.x % kXcds, part = blockIdx.x / kXcds;
     const uint32_t f = threadIdx.x & 1u, xbit = (threadIdx.x >> 1) & 1u;
     constexpr uint32_t kSamples = kScatterThreads / 4;
     for (int pass = 0; pass < 2; pass++) {
         const int lev = pass == 0 ? kLevels - 1 - (int)xcd : (int)xcd;
+        if (lev < firstLevel) continue;  // k_mlp_scatter_lds adds it
         const float* d = reinterpret_cast<const float*>(encGrad + (size_t)lev * kBatchCap);
         for (uint32_t s = part * kSamples + (threadIdx.x >> 2); s < n; s += kScatterBlocks * kSamples) {
             const float g = d[2 * (size_t)s + f];
@@ -542,9 +585,14 @@ hipError_t mlpGradients(rt_mlp* m, const float* pos, const float* target, uint32
     } else {
         (void)launch(k_fill_f32, dim3(blocks(stride, 256)), dim3(256), st, m->partial, (uint64_t)stride, 0.0f);
     }
-    if (n && store)
+    if (n && store) {
+        const int inLds = ldsLevels(m->view);
+        if (inLds)
+            (void)launch(k_mlp_scatter_lds, dim3((unsigned)inLds * 2u * kLdsParts), dim3(kLdsThreads), st, m->view, pos, n,
+                         (const float2*)m->encGrad, m->gridGrad);
         (void)launch(k_mlp_scatter, dim3(kXcds * kScatterBlocks), dim3(kScatterThreads), st, m->view, pos, n,
-                     (const float2*)m->encGrad, m->gridGrad);
+                     (const float2*)m->encGrad, inLds, m->gridGrad);
+    }
     const uint32_t rows = n ? waves : 1u;
     const uint32_t groups = (rows + kReduceGroup - 1u) / kReduceGroup;
     (void)launch(k_mlp_reduce_groups, dim3(blocks(stride, 256), groups), dim3(256), st, m->partial, rows, stride);
