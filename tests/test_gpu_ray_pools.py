@@ -1,6 +1,6 @@
-"""Where a wave hands its rays out to free lanes: ReSTIR DI's spatial pass (visibility rays of a tile's shifts in
-an LDS pool, merged afterwards in the neighbours' order) on tiles that the image only partly covers, and ray queries
-beyond the count from which a lane takes more than one ray. Bit for bit against the oracle."""
+"""Where a wave hands its rays out to free lanes: the spatial passes of ReSTIR DI and GRIS (visibility rays of a tile's
+shifts in an LDS pool, merged afterwards in the neighbours' order) on tiles that the image only partly covers, and ray
+queries beyond the count from which a lane takes more than one ray. Bit for bit against the oracle."""
 import numpy as np
 import pytest
 
@@ -11,6 +11,7 @@ torch = pytest.importorskip("torch")
 import gpuhelp  # noqa: E402
 import orc  # noqa: E402
 from test_gpu_di import run_sequence  # noqa: E402
+from test_gpu_parity import run_gris_frames  # noqa: E402
 
 rt = gpuhelp.rt
 
@@ -26,6 +27,43 @@ def test_di_spatial_on_ragged_tiles(room, size):
     for temporal, spatial in ((True, True), (False, False)):
         s = rt.di_settings(shift=0, sample=2, temporal=temporal, spatial=spatial)
         run_sequence(*room, *size, s, 2)
+
+
+@pytest.mark.parametrize("neighbors", [0, 1, 3, 4])
+@pytest.mark.parametrize("size", [(1, 1), (7, 9), (65, 17)])
+def test_gris_spatial_on_ragged_tiles(room, size, neighbors):
+    """0 to 3 neighbours go through the pool, 4 merge one by one."""
+    s = rt.settings(shift=2, temporal=True, spatial=True, cap=20, max_depth=6, neighbors=neighbors, radius=4.0)
+    assert run_gris_frames(*room, *size, s, 2) == [(0, 0, 0, 0, 0)] * 2
+
+
+@pytest.mark.parametrize("shift", [0, 1, 2])
+def test_gris_spatial_weights_that_are_not_numbers(room, shift):
+    """A shifted weight is divided by the luminance of the neighbour's F: negative, NaN and zero luminances give weights
+    that are not valid before the visibility ray, whose merge then depends on the ray, and infinite ones."""
+    hs, ds, osc = room
+    w, h, cap = 96, 40, 8
+    n = w * h
+    s = rt.settings(shift=shift, temporal=False, spatial=True, cap=cap, max_depth=5, neighbors=3, radius=6.0)
+    run = gpuhelp.GrisRun(ds, w, h)
+    cams = hs.camera(0, w, h)
+    run.gbuffer(cams[0])
+    dn, am, _, _ = osc.gbuffer(cams[0])
+    run.path_trace(cams, s)
+    run.temporal(cams, s)
+    temp = run.reservoirs(run.temp)
+    rng = np.random.default_rng(shift)
+    kind = rng.integers(0, 8, n)
+    for k, v in enumerate((-1.0, np.nan, 0.0)):
+        temp["F"][kind == k] = v
+    plane = run.temp.view(torch.float32)[12 * n:16 * n].view(n, 4)  # F and the primary ray's random state
+    plane[:, :3] = torch.from_numpy(temp["F"].copy()).to(plane.device)
+    assert not gpuhelp.compare_reservoirs(run.reservoirs(run.temp), temp).any()
+    run.spatial(cams, s)
+    out, ref = orc.reset_reservoirs(n), np.zeros((h, w, 4), np.float32)
+    osc.gris_spatial(cams, dn, am, s, temp, out, ref)
+    assert not gpuhelp.compare_reservoirs(run.reservoirs(run.resv[run.cur]), out).any()
+    assert gpuhelp.same_float(run.output(1), ref).all()
 
 
 @pytest.mark.parametrize("count", [524287, 524288, 524289, 600001])

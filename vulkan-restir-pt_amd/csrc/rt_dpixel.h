@@ -118,11 +118,12 @@ RT_DEV bool traceVisibility(const DevScene& S, TStack st, f3 from, f3 to, TraceC
 }
 
 // A wave's visibility rays, gathered in LDS so that its lanes can trace them without waiting for each other:
-// ray k runs from the origin of lane owner[k] & 63 to target[k]; an occluded one sets bit owner[k] >> 6 of that
-// lane's `blocked` word.
-template <uint32_t kRays>
+// ray k runs to target[k] from the origin of lane owner[k] & 63 or, with kOrigins, its own; an occluded one sets bit
+// owner[k] >> 6 of that lane's `blocked` word.
+template <uint32_t kRays, bool kOrigins = false>
 struct VisibilityPool {
-    float origin[3][kTileThreads];
+    static constexpr bool kOwn = kOrigins;
+    float origin[3][kOrigins ? kRays : kTileThreads];
     float target[3][kRays];
     uint32_t blocked[kTileThreads];
     uint16_t owner[kRays];
@@ -132,12 +133,13 @@ constexpr int kPoolRefill = 16;
 constexpr int kPoolStackWords = 16;  // LDS stack entries of a lane (any-hit rays keep one word each)
 
 // Appends this lane's ray (where want) to the pool; `count` is the wave's ray count. The wave is converged.
-template <uint32_t kRays>
-RT_DEV void poolAdd(VisibilityPool<kRays>& pool, uint32_t& count, bool want, f3 to, uint32_t bit) {
+template <class Pool>
+RT_DEV void poolAdd(Pool& pool, uint32_t& count, bool want, f3 to, uint32_t bit, f3 from = s3(0.0f)) {
     const unsigned long long mask = __ballot(want);
     if (want) {
         const uint32_t k = count + (uint32_t)__popcll(mask & ((1ull << threadIdx.x) - 1ull));
         pool.target[0][k] = to.x; pool.target[1][k] = to.y; pool.target[2][k] = to.z;
+        if (Pool::kOwn) { pool.origin[0][k] = from.x; pool.origin[1][k] = from.y; pool.origin[2][k] = from.z; }
         pool.owner[k] = (uint16_t)(threadIdx.x | bit << 6);
     }
     count += (uint32_t)__popcll(mask);
@@ -145,8 +147,8 @@ RT_DEV void poolAdd(VisibilityPool<kRays>& pool, uint32_t& count, bool want, f3 
 
 // Traces the pool's `count` rays (traceVisibility of each) and empties it. All 64 lanes of the one-wave
 // workgroup call it.
-template <bool kCount, uint32_t kRays>
-RT_DEV void poolTrace(const DevScene& S, TStack st, VisibilityPool<kRays>& pool, uint32_t& count, TraceCounters* ctr) {
+template <bool kCount, class Pool>
+RT_DEV void poolTrace(const DevScene& S, TStack st, Pool& pool, uint32_t& count, TraceCounters* ctr) {
     __syncthreads();
     StackSpill spill;
     WalkWork work{0, 0};
@@ -167,7 +169,7 @@ RT_DEV void poolTrace(const DevScene& S, TStack st, VisibilityPool<kRays>& pool,
             const uint32_t k = next + (uint32_t)__popcll(idle & ((1ull << threadIdx.x) - 1ull));
             if (k < count) {
                 owner = pool.owner[k];
-                const uint32_t l = owner & 63u;
+                const uint32_t l = Pool::kOwn ? k : owner & 63u;
                 const f3 from = mk3(pool.origin[0][l], pool.origin[1][l], pool.origin[2][l]);
                 const f3 to = mk3(pool.target[0][k], pool.target[1][k], pool.target[2][k]);
                 startWalk(S, w, from, normalize(to - from), RT_MIN_RAY, distance(to, from) - RT_MIN_RAY);

@@ -32,6 +32,9 @@ namespace {
 #ifndef RT_WAVES_TRACE
 #define RT_WAVES_TRACE 4
 #endif
+#ifndef RT_WAVES_SPATIAL_POOL
+#define RT_WAVES_SPATIAL_POOL 3
+#endif
 #ifndef RT_WAVES_GBUFFER
 #define RT_WAVES_GBUFFER 4
 #endif
@@ -875,10 +878,13 @@ RT_DEV float rcLightMIS(const DevScene& S, uint32_t rcType, const Surf& rcPrevSu
 // pdf_src / pdf_dst, so the next shift's target ratio is exact, as it is for a
 // fresh sample), a shift to a zero-pdf reconnection is rejected, and the M-cap
 // is left to the caller (applied once per pass after the 1/Z normalisation).
-template <bool kCount, bool kLearned = false, bool kUnbiased = false, class Dst = Resv>
-RT_DEV void reuseAndMerge(const DevScene& S, TStack st, const rt_gris_settings& set, Dst& dst, const Surf& dstPrimarySurf,
-                          const Isec& dstPrimaryIsec, f3 primDir, f3 primOri, Resv src, uint32_t& rng, TraceCounters* ctr,
-                          const rtg::GuidePix& gpx) {
+//
+// shiftOnto: src becomes the shifted sample, with the weight it has if the ray from `from` to `to` is free. Returns
+// whether the shift is valid, i.e. asks for that ray; otherwise the weight is 0.
+template <bool kCount, bool kLearned = false, bool kUnbiased = false>
+RT_DEV bool shiftOnto(const DevScene& S, TStack st, const rt_gris_settings& set, const Surf& dstPrimarySurf,
+                      const Isec& dstPrimaryIsec, f3 primDir, f3 primOri, Resv& src, f3& from, f3& to, TraceCounters* ctr,
+                      const rtg::GuidePix& gpx) {
     RcData rc;
     Surf rcPrevSurf, rcSurf;
     f3 wi = s3(0.0f), Li = s3(0.0f);
@@ -907,11 +913,9 @@ RT_DEV void reuseAndMerge(const DevScene& S, TStack st, const rt_gris_settings& 
                         isBSDFConnectible(rcPrevMat);
         }
     }
-    // The shifted sample is formed before its reconnection's visibility is traced, so that only
-    // it and the ray stay live across the traversal; an occluded or failed shift merges with
-    // weight 0 (only its M counts, as a weight-0 candidate is never picked).
     if (shiftable) {
-        const f3 visFrom = rcPrevSurf.pos, visTo = rcSurf.pos;
+        from = rcPrevSurf.pos;
+        to = rcSurf.pos;
         uint32_t rcType = flagsRcVertexType(src.flags);
         f3 LiL = s3(0.0f);
         if (!isnan(src.rcPrevSamplePdf) && src.rcPrevSamplePdf > 1e-6f) {
@@ -944,10 +948,24 @@ RT_DEV void reuseAndMerge(const DevScene& S, TStack st, const rt_gris_settings& 
         src.F = Li;
         if (src.rcPrevSamplePdf < 1e-6f || isnan(src.rcPrevSamplePdf)) src.rcPrevSamplePdf = 0.0f;
         src.resampleWeight *= dstPHat / srcPHat;
-        if (!traceVisibility<kCount>(S, st, visFrom, visTo, ctr)) src.resampleWeight = 0.0f;
     } else {
         src.resampleWeight = 0.0f;
     }
+    return shiftable;
+}
+
+// The shifted sample is formed before its reconnection's visibility is traced, so that only
+// it and the ray stay live across the traversal; an occluded or failed shift merges with
+// weight 0 (only its M counts, as a weight-0 candidate is never picked).
+template <bool kCount, bool kLearned = false, bool kUnbiased = false, class Dst = Resv>
+RT_DEV void reuseAndMerge(const DevScene& S, TStack st, const rt_gris_settings& set, Dst& dst, const Surf& dstPrimarySurf,
+                          const Isec& dstPrimaryIsec, f3 primDir, f3 primOri, Resv src, uint32_t& rng, TraceCounters* ctr,
+                          const rtg::GuidePix& gpx) {
+    f3 from, to;
+    if (shiftOnto<kCount, kLearned, kUnbiased>(S, st, set, dstPrimarySurf, dstPrimaryIsec, primDir, primOri, src, from, to,
+                                               ctr, gpx) &&
+        !traceVisibility<kCount>(S, st, from, to, ctr))
+        src.resampleWeight = 0.0f;
     if (resvIsValid(src)) resvMerge(dst, src, sample1f(rng));
     if (!kUnbiased) resvCap(dst, (float)set.cap);
 }
@@ -1098,6 +1116,60 @@ __global__ __launch_bounds__(kTileThreads, kUnbiased ? RT_WAVES_TEMPORAL_UB : RT
                                     kGuided ? gf : rtg::GuideFrame{nullptr, nullptr, nullptr});
 }
 
+// findNeighborReservoir (gris_resample_spatial.glsl:11-34) of the disk sample drawn from rng: the neighbour's pixel and
+// reservoir, if its surface is similar and the reservoir valid.
+template <bool kLearned>
+RT_DEV bool spatialNeighbor(const rt_camera& cam, const GB& g, const rt_gris_settings& set, const ResvPlanes& tempR, f2 uv,
+                            const GPix& gp, f3 pos, uint32_t& rng, int& px, int& py, Resv& nres) {
+    const f2 texel = mk2(1.0f / (float)g.W, 1.0f / (float)g.H);
+    f2 dsk = toConcentricDisk(sample2f(rng));
+    f2 nb = uv + (dsk * set.spatialRadius) * texel;
+    if (nb.x < 0.0f || nb.y < 0.0f || nb.x > 1.0f || nb.y > 1.0f) return false;
+    px = (int)(nb.x * (float)cam.filmSize[0]);
+    py = (int)(nb.y * (float)cam.filmSize[1]);
+    GPix np;
+    if (!unpackGB(texDN(g, nb), fetchAM(g, px, py), np)) return false;
+    CamRay nr = pinholeRay(cam, mk2(nb.x, 1.0f - nb.y));
+    f3 posN = nr.ori + nr.dir * (np.depth - 1e-4f);
+    if (dot(np.norm, gp.norm) < 0.9f || distance(pos, posN) > 0.4f) return false;
+    nres = resvAt<kLearned>(tempR, cam.filmSize[0], cam.filmSize[1], px, py);
+    return resvIsValid(nres);
+}
+
+// The merged reservoir stored, and the pixel shaded from it (gris_resample_spatial.glsl:100-135).
+template <bool kCount, bool kLearned, bool kUnbiased>
+RT_DEV f3 spatialShade(const DevScene& S, TStack st, const rt_gris_settings& set, Resv& resv, const ResvPlanes& thisR, size_t p,
+                       const Surf& dstPrimarySurf, const Isec& dstPrimaryIsec, const CamRay& ray, TraceCounters* ctr,
+                       const rtg::GuidePix& gpx) {
+    f3 radiance = s3(0.0f);
+    if (!resvIsValid(resv)) resvReset(resv);
+    storeResv<kLearned>(thisR, p, resv);
+    if (resvIsValid(resv) && resv.sampleCount > 0.0f && resv.rcIsec.inst != RT_INVALID_HIT) {
+        RcData rc;
+        replayHybrid<kCount>(S, st, set, dstPrimaryIsec, dstPrimarySurf, ray.dir, ray.ori, resv.flags, resv.primaryRng,
+                             rc, ctr, gpx);
+        if (rc.rcPrevIsec.inst != RT_INVALID_HIT) {
+            Surf rcPrevSurf, rcSurf;
+            if (rc.rcPrevIsec.inst == RT_SPECIAL_HIT) rcPrevSurf = dstPrimarySurf;
+            else loadSurfaceInfo(S, rc.rcPrevIsec, rcPrevSurf);
+            loadSurfaceInfo(S, resv.rcIsec, rcSurf);
+            f3 wi = normalize(rcSurf.pos - rcPrevSurf.pos);
+            float misW = 1.0f;
+            if (kUnbiased) {
+                const float gj = fabsf(dot(rcSurf.norm, wi)) / square(distance(rcPrevSurf.pos, rcSurf.pos));
+                misW = rcLightMIS(S, flagsRcVertexType(resv.flags), rcPrevSurf, rc.rcPrevWo, rcSurf, wi, gj);
+            }
+            f3 Li = reconnectLi(S, resv, kUnbiased ? resv.rcLi * misW : resv.rcLi, rcPrevSurf, rcSurf, wi, rc,
+                                kUnbiased);
+            float pHat = kLearned ? luminance(reconnectLi(S, resv, kUnbiased ? targetRcLi(resv) * misW : targetRcLi(resv),
+                                                          rcPrevSurf, rcSurf, wi, rc, kUnbiased))
+                                  : luminance(Li);
+            if (!isBlack(Li) && !hasNan(Li)) radiance = Li / pHat * resv.resampleWeight / resv.sampleCount;
+        }
+    }
+    return clampColor(radiance);
+}
+
 // gris_resample_spatial.glsl:11-135 and gris_resample_spatial.comp accumulation
 template <bool kCount, bool kLearned, bool kUnbiased = false>
 RT_DEV void spatialPixel(const DevScene& S, const rt_camera& cam, const GB& g, const rt_gris_settings& set,
@@ -1130,21 +1202,10 @@ RT_DEV void spatialPixel(const DevScene& S, const rt_camera& cam, const GB& g, c
         LdsResv dstL{dstSlot, resv.sampleCount, resv.resampleWeight};
         if constexpr (kDstInLds) storeStream(dstSlot, resv);
         if (set.spatialReuse) {
-            f2 texel = mk2(1.0f / (float)g.W, 1.0f / (float)g.H);
             for (uint32_t i = 0; i < set.spatialNeighbors; i++) {
-                f2 dsk = toConcentricDisk(sample2f(rng));
-                f2 nb = uv + (dsk * set.spatialRadius) * texel;
-                // findNeighborReservoir (gris_resample_spatial.glsl:11-34)
-                if (nb.x < 0.0f || nb.y < 0.0f || nb.x > 1.0f || nb.y > 1.0f) continue;
-                int px = (int)(nb.x * (float)cam.filmSize[0]);
-                int py = (int)(nb.y * (float)cam.filmSize[1]);
-                GPix np;
-                if (!unpackGB(texDN(g, nb), fetchAM(g, px, py), np)) continue;
-                CamRay nr = pinholeRay(cam, mk2(nb.x, 1.0f - nb.y));
-                f3 posN = nr.ori + nr.dir * (np.depth - 1e-4f);
-                if (dot(np.norm, gp.norm) < 0.9f || distance(pos, posN) > 0.4f) continue;
-                Resv nres = resvAt<kLearned>(tempR, cam.filmSize[0], cam.filmSize[1], px, py);
-                if (resvIsValid(nres)) {
+                int px, py;
+                Resv nres;
+                if (spatialNeighbor<kLearned>(cam, g, set, tempR, uv, gp, pos, rng, px, py, nres)) {
                     if constexpr (kDstInLds)
                         reuseAndMerge<kCount, kLearned, kUnbiased>(S, st, set, dstL, dstPrimarySurf, dstPrimaryIsec,
                                                                     ray.dir, ray.ori, nres, rng, ctr, gpx);
@@ -1180,32 +1241,8 @@ RT_DEV void spatialPixel(const DevScene& S, const rt_camera& cam, const GB& g, c
             }
             resvCap(resv, (float)set.cap);
         }
-        if (!resvIsValid(resv)) resvReset(resv);
-        storeResv<kLearned>(thisR, p, resv);
-        if (resvIsValid(resv) && resv.sampleCount > 0.0f && resv.rcIsec.inst != RT_INVALID_HIT) {
-            RcData rc;
-            replayHybrid<kCount>(S, st, set, dstPrimaryIsec, dstPrimarySurf, ray.dir, ray.ori, resv.flags, resv.primaryRng,
-                                 rc, ctr, gpx);
-            if (rc.rcPrevIsec.inst != RT_INVALID_HIT) {
-                Surf rcPrevSurf, rcSurf;
-                if (rc.rcPrevIsec.inst == RT_SPECIAL_HIT) rcPrevSurf = dstPrimarySurf;
-                else loadSurfaceInfo(S, rc.rcPrevIsec, rcPrevSurf);
-                loadSurfaceInfo(S, resv.rcIsec, rcSurf);
-                f3 wi = normalize(rcSurf.pos - rcPrevSurf.pos);
-                float misW = 1.0f;
-                if (kUnbiased) {
-                    const float gj = fabsf(dot(rcSurf.norm, wi)) / square(distance(rcPrevSurf.pos, rcSurf.pos));
-                    misW = rcLightMIS(S, flagsRcVertexType(resv.flags), rcPrevSurf, rc.rcPrevWo, rcSurf, wi, gj);
-                }
-                f3 Li = reconnectLi(S, resv, kUnbiased ? resv.rcLi * misW : resv.rcLi, rcPrevSurf, rcSurf, wi, rc,
-                                    kUnbiased);
-                float pHat = kLearned ? luminance(reconnectLi(S, resv, kUnbiased ? targetRcLi(resv) * misW : targetRcLi(resv),
-                                                              rcPrevSurf, rcSurf, wi, rc, kUnbiased))
-                                      : luminance(Li);
-                if (!isBlack(Li) && !hasNan(Li)) radiance = Li / pHat * resv.resampleWeight / resv.sampleCount;
-            }
-        }
-        radiance = clampColor(radiance);
+        radiance = spatialShade<kCount, kLearned, kUnbiased>(S, st, set, resv, thisR, p, dstPrimarySurf, dstPrimaryIsec, ray,
+                                                             ctr, gpx);
     }
     accumulate(indirectOut, p, radiance, cam.frameIndex);
 }
@@ -1220,6 +1257,107 @@ __global__ __launch_bounds__(kTileThreads, kUnbiased ? RT_WAVES_SPATIAL_UB : RT_
                                               laneStack(stk), ctr,
                                               kGuided ? gf : rtg::GuideFrame{nullptr, nullptr, nullptr},
                                               StreamSlot{dstWords + threadIdx.x, (uint32_t)kTileThreads});
+}
+
+// The same pass with the luminance target, the reference's weights and BSDF sampling for up to kPoolNeighbors
+// neighbours, its visibility rays traced from a pool as in ReSTIR DI's spatial pass: all shifts first, then the rays by
+// whichever lane is free, the merges last in the neighbours' order and the picked shift formed again. A merge draws its
+// random number if the shifted weight is valid, and an occluded shift's weight 0 is, so a weight that is not valid
+// before its ray asks for the pool to be traced at once. A weight of 0 merges the same whether its ray is blocked or
+// not, so only the counting build traces that ray. Bound by the instructions of divergent traversal: one merge after
+// another runs at 16 of 64 lanes. The 1080p terrain frame takes 3.83 ms with this kernel and 4.04 without it, a 64x64
+// view of the box room 0.64 and 0.69. Its 12.4 KB of LDS let 12 waves share a compute unit, hence 3 waves per SIMD:
+// registers for 4 (more spilling, no more waves) give 3.93 ms. A fourth neighbour's rays and weights would cost
+// another of those waves, so more neighbours go to k_gris_spatial.
+constexpr uint32_t kPoolNeighbors = 3;
+template <bool kCount>
+__global__ __launch_bounds__(kTileThreads, RT_WAVES_SPATIAL_POOL) void k_gris_spatial_pool(
+    DevScene S, rt_camera cam, GB g, rt_gris_settings set, ResvPlanes tempR, ResvPlanes thisR, float* indirectOut,
+    TraceCounters* ctr) {
+    __shared__ StackLDS<kTileThreads> stk;
+    __shared__ VisibilityPool<kPoolNeighbors * kTileThreads, true> pool;
+    __shared__ float weights[kPoolNeighbors][kTileThreads], counts[kPoolNeighbors][kTileThreads];
+    PIXEL_INDEX
+    const TStack st = laneStack(stk);
+    const uint32_t lane = threadIdx.x;
+    const rtg::GuidePix gpx = rtg::noGuide();
+    const bool inside = x < g.W && y < g.H;
+    const size_t p = (size_t)y * g.W + x;
+    const f2 uv = pixelUV(x, y, g.W, g.H);
+    GPix gp;
+    const bool surface = inside && unpackGB(texDNCentre(g, x, y), fetchAM(g, (int)x, (int)y), gp);
+    const CamRay ray = pinholeRay(cam, mk2(uv.x, 1.0f - uv.y));
+    Surf dstPrimarySurf;
+    Isec dstPrimaryIsec; dstPrimaryIsec.inst = RT_SPECIAL_HIT; dstPrimaryIsec.b1 = uv.x; dstPrimaryIsec.b2 = uv.y;
+    dstPrimaryIsec.prim = 0u;
+    if (surface) {
+        dstPrimarySurf.pos = ray.ori + ray.dir * (gp.depth - 1e-4f);
+        dstPrimarySurf.norm = gp.norm; dstPrimarySurf.albedo = gp.albedo;
+        dstPrimarySurf.matIndex = (uint32_t)(gp.matMeshId >> 16); dstPrimarySurf.isLight = false;
+    }
+    const uint32_t rng0 = makeSeedPix(cam.seed, x, y) ^ 2u;
+    uint32_t rng = rng0, found = 0, valid = 0, count = 0;  // bit i: neighbour i merges / its weight is valid
+    if (set.spatialReuse) {
+        pool.blocked[lane] = 0u;
+        for (uint32_t i = 0; i < set.spatialNeighbors; i++) {
+            bool want = false, late = false;
+            f3 from = s3(0.0f), to = s3(0.0f);
+            Resv nres;
+            int px, py;
+            if (surface && spatialNeighbor<false>(cam, g, set, tempR, uv, gp, dstPrimarySurf.pos, rng, px, py, nres)) {
+                found |= 1u << i;
+                counts[i][lane] = nres.sampleCount;
+                const bool shifted = shiftOnto<kCount>(S, st, set, dstPrimarySurf, dstPrimaryIsec, ray.dir, ray.ori, nres,
+                                                       from, to, ctr, gpx);
+                weights[i][lane] = nres.resampleWeight;
+                want = shifted && (kCount || nres.resampleWeight != 0.0f);
+                late = !resvIsValid(nres);
+                if (!late) valid |= 1u << i;
+            }
+            poolAdd(pool, count, want, to, i, from);
+            if (__ballot(late) != 0ull) {
+                poolTrace<kCount>(S, st, pool, count, ctr);
+                if (late && (pool.blocked[lane] >> i) & 1u) valid |= 1u << i;
+            }
+            if ((valid >> i) & 1u) (void)sample1f(rng);  // the merge's random number
+        }
+        poolTrace<kCount>(S, st, pool, count, ctr);
+    }
+    f3 radiance = s3(0.0f);
+    if (surface) {
+        Resv resv = loadResv(tempR, p);
+        if (found) {
+            const uint32_t blocked = pool.blocked[lane];
+            float m = resv.sampleCount, sum = resv.resampleWeight;
+            uint32_t pick = 0u;
+            bool picked = false;
+            rng = rng0;
+            for (uint32_t i = 0; i < set.spatialNeighbors; i++) {
+                const uint32_t before = rng;
+                (void)sample2f(rng);
+                if (!((found >> i) & 1u)) continue;
+                if ((valid >> i) & 1u) {
+                    const float u = sample1f(rng);
+                    const float w = (blocked >> i) & 1u ? 0.0f : weights[i][lane];
+                    m += counts[i][lane];
+                    sum += w;
+                    if (u * sum < w) { pick = before; picked = true; }
+                }
+                if (m > (float)set.cap) { sum *= (float)set.cap / m; m = (float)set.cap; }  // resvCap
+            }
+            Resv nres;
+            int px, py;
+            if (picked && spatialNeighbor<false>(cam, g, set, tempR, uv, gp, dstPrimarySurf.pos, pick, px, py, nres)) {
+                f3 from, to;
+                (void)shiftOnto<false>(S, st, set, dstPrimarySurf, dstPrimaryIsec, ray.dir, ray.ori, nres, from, to, ctr, gpx);
+                resv = nres;
+            }
+            resv.sampleCount = m;
+            resv.resampleWeight = sum;
+        }
+        radiance = spatialShade<kCount, false, false>(S, st, set, resv, thisR, p, dstPrimarySurf, dstPrimaryIsec, ray, ctr, gpx);
+    }
+    if (inside) accumulate(indirectOut, p, radiance, cam.frameIndex);
 }
 
 // ---- Batched views ---------------------------------------------------------------------------
@@ -1850,6 +1988,14 @@ hipError_t launchGrisTemporal(const rt_device_scene* s, const rt_camera* cams, c
 hipError_t launchGrisSpatial(const rt_device_scene* s, const rt_camera* cams, const rt_frame& f,
                              const rt_gris_settings& set, hipStream_t stream) {
     GB g = makeGB(f.depthNormal, f.albedoMatId, f.motionVector, f.width, f.height);
+    if (set.targetFunction == 0u && set.unbiasedReuse == 0u && set.guidedProposal == 0u &&
+        set.spatialNeighbors <= kPoolNeighbors) {
+        TraceCounters* ctr = gCountersEnabled ? counterBuffer() : nullptr;
+        (void)launch(gCountersEnabled ? k_gris_spatial_pool<true> : k_gris_spatial_pool<false>, tileGrid(f.width, f.height),
+                     kTileThreads, stream, s->dev, cams[0], g, set, planes(f.grisReservoirTemp, f.width, f.height),
+                     planes(f.grisReservoir, f.width, f.height), f.indirectOutput, ctr);
+        return hipGetLastError();
+    }
     RT_DISPATCH_LUG(k_gris_spatial, set.targetFunction == 1u, set.unbiasedReuse == 1u, set.guidedProposal == 1u,
                     tileGrid(f.width, f.height),
                    kTileThreads, stream, s->dev,
