@@ -1,6 +1,8 @@
 """Where a wave hands its rays out to free lanes: the spatial passes of ReSTIR DI and GRIS (visibility rays of a tile's
 shifts in an LDS pool, merged afterwards in the neighbours' order) on tiles that the image only partly covers, and ray
 queries beyond the count from which a lane takes more than one ray. Bit for bit against the oracle."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -10,6 +12,7 @@ torch = pytest.importorskip("torch")
 
 import gpuhelp  # noqa: E402
 import orc  # noqa: E402
+from test_gpu_batch import make_view  # noqa: E402
 from test_gpu_di import run_sequence  # noqa: E402
 from test_gpu_parity import run_gris_frames  # noqa: E402
 
@@ -64,6 +67,37 @@ def test_gris_spatial_weights_that_are_not_numbers(room, shift):
     osc.gris_spatial(cams, dn, am, s, temp, out, ref)
     assert not gpuhelp.compare_reservoirs(run.reservoirs(run.resv[run.cur]), out).any()
     assert gpuhelp.same_float(run.output(1), ref).all()
+
+
+@pytest.mark.parametrize("neighbors", [(3, 2, 0), (3, 5, 1)])
+def test_batched_gris_spatial(room, neighbors):
+    """A batch takes the pool if all its views do; a graph built for one choice is rebuilt for the other."""
+    hs, ds, _ = room
+    sizes = [(64, 17), (7, 9), (40, 40)]
+    b = C.c_void_p()
+    L = rt.core()
+    rt.check(L.rt_batch_create(len(sizes), C.byref(b)), "batch create")
+    try:
+        t = rt.BatchTuning()
+        t.graph = 1
+        rt.check(L.rt_batch_set_tuning(b, C.byref(t)), "tuning")
+        single, batched = ([gpuhelp.GrisRun(ds, *z) for z in sizes] for _ in range(2))
+        for frame, ns in enumerate(((1, 2, 3), neighbors, neighbors)):
+            views = (rt.View * len(sizes))()
+            for i, z in enumerate(sizes):
+                s = rt.settings(shift=2, temporal=True, spatial=True, cap=20, max_depth=5, neighbors=ns[i], radius=5.0)
+                cams = hs.camera(frame, *z)
+                single[i].frame(cams, s)
+                views[i] = make_view(batched[i], ds, cams, s)
+            rt.check(L.rt_batch_frame(b, views, len(sizes), gpuhelp.stream()), "batch frame")
+            torch.cuda.synchronize()
+            for a, z in zip(single, batched):
+                assert not gpuhelp.compare_reservoirs(a.reservoirs(a.resv[a.cur]), z.reservoirs(z.resv[z.cur])).any()
+                assert gpuhelp.same_float(a.output(1), z.output(1)).all()
+                a.flip()
+                z.flip()
+    finally:
+        L.rt_batch_destroy(b)
 
 
 @pytest.mark.parametrize("count", [524287, 524288, 524289, 600001])

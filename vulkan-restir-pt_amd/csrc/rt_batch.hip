@@ -39,7 +39,8 @@ hipError_t launchBatchGBuffer(const void* descs, uint32_t numViews, uint32_t tot
 hipError_t launchBatchPathTrace(const void* descs, uint32_t numViews, uint32_t persistentGroups, bool guided,
                                 uint32_t waveVariant, hipStream_t stream);
 hipError_t launchBatchReuse(const void* descs, uint32_t numViews, uint32_t totalTiles, uint32_t xcdSwizzle,
-                            bool learned, bool unbiased, bool guided, hipStream_t stream);
+                            bool learned, bool unbiased, bool guided, bool pooled, hipStream_t stream);
+bool pooledSpatial(const rt_gris_settings& set);
 hipError_t launchLearnedRefresh(const rt_device_scene*, rt_mlp*, const rt_camera*, const rt_frame&, hipStream_t);
 hipError_t mlpGradients(rt_mlp* m, const float* pos, const float* target, uint32_t n, float* loss, hipStream_t st);
 hipError_t mlpAdam(rt_mlp* m, hipStream_t st);
@@ -133,7 +134,7 @@ uint32_t formOf(const rt_gris_settings& s) {
     return (s.targetFunction ? 1u : 0u) | (s.unbiasedReuse ? 2u : 0u) | (s.guidedProposal ? 4u : 0u);
 }
 
-struct Group { uint32_t first, count, form; uint64_t tiles; };
+struct Group { uint32_t first, count, form; uint64_t tiles; bool pooled; };  // pooled: pooledSpatial of every view
 
 // The frame's kernel launches (launched, or recorded while a recorder is
 // installed): per form G-buffer, proposal refreshes, one persistent path trace,
@@ -165,7 +166,7 @@ hipError_t frameLaunches(rt_batch* b, const rt_view* views, uint32_t n, const st
         }
     for (const Group& gr : groups) {
         e = rti::launchBatchReuse(descs + b->descBytes * gr.first, gr.count, (uint32_t)gr.tiles, t.xcdSwizzle,
-                                  (gr.form & 1u) != 0u, (gr.form & 2u) != 0u, (gr.form & 4u) != 0u, stream);
+                                  (gr.form & 1u) != 0u, (gr.form & 2u) != 0u, (gr.form & 4u) != 0u, gr.pooled, stream);
         if (e != hipSuccess) return e;
     }
     // one training step per network (rt_mlp_train_frame, rt_gris_guide_train)
@@ -221,7 +222,7 @@ rt_status frame(rt_batch* b, const rt_view* views, uint32_t n, const rt_batch_tu
     for (uint32_t j = 0; j < n; j++) {
         const rt_view& v = views[order[j]];
         const uint32_t form = formOf(v.settings);
-        if (groups.empty() || groups.back().form != form) groups.push_back(Group{j, 0u, form, 0ull});
+        if (groups.empty() || groups.back().form != form) groups.push_back(Group{j, 0u, form, 0ull, true});
         Group& gr = groups.back();
         rti::batchFillDesc(stage + b->descBytes * j, v.scene, v.cams, v.frame, v.settings, (uint32_t)gr.tiles,
                            b->queues + j, qShift, (uint32_t)pixels);
@@ -229,6 +230,7 @@ rt_status frame(rt_batch* b, const rt_view* views, uint32_t n, const rt_batch_tu
         maxDepth = std::max(maxDepth, v.settings.maxDepth);
         gr.tiles += rti::batchViewTiles(v.frame);
         gr.count++;
+        gr.pooled = gr.pooled && rti::pooledSpatial(v.settings);
         // a launch's grid (tiles rounded up to 8 chunks) stays within 2^26 64-lane workgroups
         if (gr.tiles > kMaxTiles) return invalid("too many tiles in one batch");
         anyGuided = anyGuided || v.settings.guidedProposal;

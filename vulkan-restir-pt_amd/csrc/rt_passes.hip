@@ -1266,19 +1266,20 @@ __global__ __launch_bounds__(kTileThreads, kUnbiased ? RT_WAVES_SPATIAL_UB : RT_
 // before its ray asks for the pool to be traced at once. A weight of 0 merges the same whether its ray is blocked or
 // not, so only the counting build traces that ray. Bound by the instructions of divergent traversal: one merge after
 // another runs at 16 of 64 lanes. The 1080p terrain frame takes 3.83 ms with this kernel and 4.04 without it, a 64x64
-// view of the box room 0.64 and 0.69. Its 12.4 KB of LDS let 12 waves share a compute unit, hence 3 waves per SIMD:
+// view of the box room 0.64 and 0.69, sixteen views in one batch 5.17 and 5.36. Its 12.4 KB of LDS let 12 waves share a compute unit, hence 3 waves per SIMD:
 // registers for 4 (more spilling, no more waves) give 3.93 ms. A fourth neighbour's rays and weights would cost
 // another of those waves, so more neighbours go to k_gris_spatial.
 constexpr uint32_t kPoolNeighbors = 3;
+struct SpatialPool {
+    VisibilityPool<kPoolNeighbors * kTileThreads, true> rays;
+    float weights[kPoolNeighbors][kTileThreads], counts[kPoolNeighbors][kTileThreads];  // of a lane's shifts
+};
 template <bool kCount>
-__global__ __launch_bounds__(kTileThreads, RT_WAVES_SPATIAL_POOL) void k_gris_spatial_pool(
-    DevScene S, rt_camera cam, GB g, rt_gris_settings set, ResvPlanes tempR, ResvPlanes thisR, float* indirectOut,
-    TraceCounters* ctr) {
-    __shared__ StackLDS<kTileThreads> stk;
-    __shared__ VisibilityPool<kPoolNeighbors * kTileThreads, true> pool;
-    __shared__ float weights[kPoolNeighbors][kTileThreads], counts[kPoolNeighbors][kTileThreads];
-    PIXEL_INDEX
-    const TStack st = laneStack(stk);
+RT_DEV void spatialPoolTile(const DevScene& S, const rt_camera& cam, const GB& g, const rt_gris_settings& set,
+                            const ResvPlanes& tempR, const ResvPlanes& thisR, float* indirectOut, uint32_t x, uint32_t y,
+                            TStack st, SpatialPool& tile, TraceCounters* ctr) {
+    auto& pool = tile.rays;
+    auto &weights = tile.weights, &counts = tile.counts;
     const uint32_t lane = threadIdx.x;
     const rtg::GuidePix gpx = rtg::noGuide();
     const bool inside = x < g.W && y < g.H;
@@ -1358,6 +1359,15 @@ __global__ __launch_bounds__(kTileThreads, RT_WAVES_SPATIAL_POOL) void k_gris_sp
         radiance = spatialShade<kCount, false, false>(S, st, set, resv, thisR, p, dstPrimarySurf, dstPrimaryIsec, ray, ctr, gpx);
     }
     if (inside) accumulate(indirectOut, p, radiance, cam.frameIndex);
+}
+template <bool kCount>
+__global__ __launch_bounds__(kTileThreads, RT_WAVES_SPATIAL_POOL) void k_gris_spatial_pool(
+    DevScene S, rt_camera cam, GB g, rt_gris_settings set, ResvPlanes tempR, ResvPlanes thisR, float* indirectOut,
+    TraceCounters* ctr) {
+    __shared__ StackLDS<kTileThreads> stk;
+    __shared__ SpatialPool tile;
+    PIXEL_INDEX
+    spatialPoolTile<kCount>(S, cam, g, set, tempR, thisR, indirectOut, x, y, laneStack(stk), tile, ctr);
 }
 
 // ---- Batched views ---------------------------------------------------------------------------
@@ -1470,6 +1480,18 @@ __global__ __launch_bounds__(kTileThreads, kUnbiased ? RT_WAVES_SPATIAL_UB : RT_
                                               laneStack(stk), ctr,
                                               kGuided ? D.gf : rtg::GuideFrame{nullptr, nullptr, nullptr},
                                               StreamSlot{dstWords + threadIdx.x, (uint32_t)kTileThreads});
+}
+
+// Views whose settings k_gris_spatial_pool takes.
+template <bool kCount>
+__global__ __launch_bounds__(kTileThreads, RT_WAVES_SPATIAL_POOL) void k_gris_spatial_pool_batch(
+    const ViewDesc* __restrict__ V, uint32_t numViews, uint32_t totalTiles, uint32_t swz, TraceCounters* ctr) {
+    __shared__ StackLDS<kTileThreads> stk;
+    __shared__ SpatialPool tile;
+    uint32_t v, x, y;
+    if (!batchPixel(V, numViews, totalTiles, swz, v, x, y)) return;  // the whole workgroup
+    const ViewDesc& D = V[v];
+    spatialPoolTile<kCount>(D.S, D.cam, D.g, D.set, D.temp, D.cur, D.indirectOut, x, y, laneStack(stk), tile, ctr);
 }
 
 // ---- Wavefront variant of the batched path trace: material-sorted shading ----
@@ -1985,15 +2007,19 @@ hipError_t launchGrisTemporal(const rt_device_scene* s, const rt_camera* cams, c
     return hipGetLastError();
 }
 
+// Whether k_gris_spatial_pool (one view or a batch of such views) takes these settings.
+bool pooledSpatial(const rt_gris_settings& set) {
+    return set.targetFunction == 0u && set.unbiasedReuse == 0u && set.guidedProposal == 0u &&
+           set.spatialNeighbors <= kPoolNeighbors;
+}
+
 hipError_t launchGrisSpatial(const rt_device_scene* s, const rt_camera* cams, const rt_frame& f,
                              const rt_gris_settings& set, hipStream_t stream) {
     GB g = makeGB(f.depthNormal, f.albedoMatId, f.motionVector, f.width, f.height);
-    if (set.targetFunction == 0u && set.unbiasedReuse == 0u && set.guidedProposal == 0u &&
-        set.spatialNeighbors <= kPoolNeighbors) {
-        TraceCounters* ctr = gCountersEnabled ? counterBuffer() : nullptr;
-        (void)launch(gCountersEnabled ? k_gris_spatial_pool<true> : k_gris_spatial_pool<false>, tileGrid(f.width, f.height),
-                     kTileThreads, stream, s->dev, cams[0], g, set, planes(f.grisReservoirTemp, f.width, f.height),
-                     planes(f.grisReservoir, f.width, f.height), f.indirectOutput, ctr);
+    if (pooledSpatial(set)) {
+        RT_DISPATCH(k_gris_spatial_pool, tileGrid(f.width, f.height), kTileThreads, stream, s->dev, cams[0], g, set,
+                    planes(f.grisReservoirTemp, f.width, f.height), planes(f.grisReservoir, f.width, f.height),
+                    f.indirectOutput);
         return hipGetLastError();
     }
     RT_DISPATCH_LUG(k_gris_spatial, set.targetFunction == 1u, set.unbiasedReuse == 1u, set.guidedProposal == 1u,
@@ -2160,12 +2186,16 @@ hipError_t launchBatchWavefront(const void* descs, uint32_t numViews, uint32_t t
 }
 
 hipError_t launchBatchReuse(const void* descs, uint32_t numViews, uint32_t totalTiles, uint32_t xcdSwizzle,
-                            bool learned, bool unbiased, bool guided, hipStream_t stream) {
+                            bool learned, bool unbiased, bool guided, bool pooled, hipStream_t stream) {
     const ViewDesc* V = reinterpret_cast<const ViewDesc*>(descs);
     const uint32_t swz = xcdSwizzle;
     const dim3 grid = batchTileGrid(totalTiles, swz);
     RT_DISPATCH_LUG(k_gris_temporal_batch, learned, unbiased, guided, grid, kTileThreads, stream, V, numViews,
                     totalTiles, swz);
+    if (pooled) {
+        RT_DISPATCH(k_gris_spatial_pool_batch, grid, kTileThreads, stream, V, numViews, totalTiles, swz);
+        return hipGetLastError();
+    }
     RT_DISPATCH_LUG(k_gris_spatial_batch, learned, unbiased, guided, grid, kTileThreads, stream, V, numViews,
                     totalTiles, swz);
     return hipGetLastError();
