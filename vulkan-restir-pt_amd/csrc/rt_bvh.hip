@@ -979,8 +979,8 @@ bool buildLBVH(rt_device_scene* s, const std::vector<uint32_t>& instPrimOffset, 
     }
     for (int k = 0; k < 3; k++)
         if (ev[k]) (void)hipEventDestroy(ev[k]);
-    // a 4-wide node pushes at most three children: the stack never holds more
-    // than 3 (depth - 1) entries
+    // a 4-wide node leaves at most three children on the stack, and the one
+    // descended into passes through it: never more than 3 depth + 1 entries
     if (ok && 3 * (uint64_t)s->bvh4Depth + 1 > RT_MAX_STACK) {
         setError("BVH depth " + std::to_string(s->bvh4Depth) + " exceeds the traversal stack");
         return false;
