@@ -150,3 +150,32 @@ def test_gbuffer_without_near_plane(near):
         run.gbuffer(cam)
         for got, want in zip(run.gbuffer_host(), osc.gbuffer(cam)[:3]):
             assert np.array_equal(got.view(np.uint8), want.view(np.uint8))
+
+
+@pytest.mark.parametrize("tmin", [1e-4, 0.0, -1.0])
+@pytest.mark.parametrize("scene", ["room", "one sliver", "slivers"])
+def test_counted_visits(scene, tmin):
+    """Nodes, triangles and rays of the counting builds, as the oracle counts them."""
+    print(f"[gpu] counted visits, {scene}, tmin {tmin}", flush=True)
+    g = np.random.default_rng(11)
+    if scene == "room":
+        keep = rt.HostScene(0, 1)
+        a = keep.arrays
+    else:
+        a, keep = light_scene(slivers(1 if scene == "one sliver" else 700, g))
+    ds, osc = rt.DeviceScene(a), orc.OracleScene(a)
+    tris = osc.world_tris()[0].reshape(-1, 3, 3)
+    rays = gpuhelp.random_rays(4097, -1.0, 1.5, seed=12, tmin=tmin)
+    if tmin >= 0:  # else entry distances of -0 and 0, which the counted order keeps apart, precede a hit
+        rays[::2, :3] = tris[g.integers(0, len(tris), 2049)].mean(axis=1)
+    rt.check(rt.core().rt_counters_enable(1), "counters")
+    try:
+        for mode in (0, 1):
+            out = np.zeros(3, np.uint64)
+            rt.check(rt.core().rt_counters_read(out.ctypes.data, 1), "read")
+            gpuhelp.gpu_trace(ds, rays, mode)
+            rt.check(rt.core().rt_counters_read(out.ctypes.data, 1), "read")
+            st = osc.trace(rays, mode)[4]
+            assert (out[0], out[1], out[2]) == (st[1], st[2], st[0]), f"mode {mode}"
+    finally:
+        rt.core().rt_counters_enable(0)

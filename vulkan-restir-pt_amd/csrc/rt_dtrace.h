@@ -27,14 +27,14 @@
 // Per lane: a short stack in LDS (strided by the block size so a wave's pushes
 // and pops hit distinct banks) that spills to a private array for deep trees.
 // Closest-hit traversal keeps each entry's distance beside it (spilled entries: its
-// top 16 bits, i.e. rounded toward zero; one that is not positive as -inf) and drops
-// a popped node that lies beyond the closest hit found since it was pushed. That
-// changes no result: a node's box contains its children's boxes, and the slab
-// distances are monotone in the bounds under IEEE rounding, so every child of such a
-// node would fail its own box test against the same closest hit. The counting builds
-// count the visits of the order that the oracle specifies, which keeps 16 bits of
-// every distance and never drops a node's nearest internal child; the plain builds
-// visit at most those nodes.
+// top 16 bits, i.e. rounded toward zero; a negative one as -inf) and drops a popped
+// node that lies beyond the closest hit found since it was pushed. That changes no
+// result: a node's box contains its children's boxes, and the slab distances are
+// monotone in the bounds under IEEE rounding, so every child of such a node would
+// fail its own box test against the same closest hit. The counting builds count the
+// visits of the order that the oracle specifies, which keeps 16 bits of every
+// distance and never drops a node's nearest internal child; the plain builds visit
+// at most those nodes.
 // Leaves hold one triangle, tested with the watertight algorithm of Woop,
 // Benthin and Wald (JCGT 2013) including its double-precision fallback. Box
 // tests use (bound - o) * (1 / d) with IEEE minNum/maxNum so that 0 * inf slabs
@@ -182,11 +182,11 @@ RT_DEV unsigned long long pushKeySigned(bool h, float t, uint32_t ref) {
     const uint32_t rank = (b >> 31) ? ~b : b | 0x80000000u;
     return h ? (unsigned long long)(ref >> 31) << 32 | (uint32_t)~rank : ~0ull;
 }
-// What the stack keeps of such a key: a positive distance, else -inf, which is never beyond a hit (a negative
-// distance cut to its top 16 bits would be a greater one).
+// What the stack keeps of such a key: the distance, or -inf, never beyond a hit, for a leaf or a negative one (which
+// would be a greater one once cut to its top 16 bits).
 RT_DEV uint32_t storedKey(unsigned long long k) {
     const uint32_t rank = ~(uint32_t)k;
-    return (k >> 32) == 0u && rank > 0x80000000u ? rank & 0x7fffffffu : 0xff800000u;
+    return (k >> 32) == 0u && rank >= 0x80000000u ? rank & 0x7fffffffu : 0xff800000u;
 }
 template <class Key>
 RT_DEV void order2(Key& ka, uint32_t& ra, Key& kb, uint32_t& rb) {
@@ -309,7 +309,8 @@ RT_DEV void walk(const DevScene& S, Walk& w, bool skipLights, TStack st, StackSp
             bool h1 = slabHit(r, nx.y, ny.y, nz.y, fx.y, fy.y, fz.y, tBest, t1);
             bool h2 = slabHit(r, nx.z, ny.z, nz.z, fx.z, fy.z, fz.z, tBest, t2);
             bool h3 = slabHit(r, nx.w, ny.w, nz.w, fx.w, fy.w, fz.w, tBest, t3);
-            if (r.flat) {
+            // (counted visits are those of min and max, also for the box of the unused child of a one-leaf tree)
+            if (kCount || r.flat) {
                 h0 = slabHitFlat(r, nx.x, ny.x, nz.x, fx.x, fy.x, fz.x, tBest, t0) & (c0 != RT_EMPTY);
                 h1 = slabHitFlat(r, nx.y, ny.y, nz.y, fx.y, fy.y, fz.y, tBest, t1) & (c1 != RT_EMPTY);
                 h2 = slabHitFlat(r, nx.z, ny.z, nz.z, fx.z, fy.z, fz.z, tBest, t2) & (c2 != RT_EMPTY);
@@ -329,14 +330,14 @@ RT_DEV void walk(const DevScene& S, Walk& w, bool skipLights, TStack st, StackSp
                 order4(k3, c3, k2, c2, k1, c1, k0, c0);
                 key[0] = storedKey(k3); key[1] = storedKey(k2); key[2] = storedKey(k1); key[3] = storedKey(k0);
             }
+            const uint32_t cs[4] = {c3, c2, c1, c0};
             if (kCount && kKeep) {
                 // the counted order visits a node's nearest internal child without a distance check: the
-                // last entry whose key is not a leaf's
+                // last entry that is not a leaf
 #pragma unroll
                 for (int q = 0; q < 4; q++)
-                    if (q < n && !(key[q] >> 31) && (q + 1 == n || (key[q + 1 < 4 ? q + 1 : 3] >> 31))) { key[q] |= RT_LEAF; break; }
+                    if (q < n && !(cs[q] >> 31) && (q + 1 == n || (cs[q + 1 < 4 ? q + 1 : 3] >> 31))) { key[q] = 0xff800000u; break; }
             }
-            const uint32_t cs[4] = {c3, c2, c1, c0};
             if (sp + 4 <= kCap) {  // the missed children land above the top
                 LdsWord* e = st.lds + sp * entry;
 #pragma unroll
