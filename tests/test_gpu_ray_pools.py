@@ -1,6 +1,6 @@
 """Where a wave hands its rays out to free lanes: the spatial passes of ReSTIR DI and GRIS (visibility rays of a tile's
 shifts in an LDS pool, merged afterwards in the neighbours' order) on tiles that the image only partly covers, and ray
-queries beyond the count from which a lane takes more than one ray. Bit for bit against the oracle."""
+queries of more waves than the device holds at once. Bit for bit against the oracle."""
 import ctypes as C
 
 import numpy as np
@@ -101,7 +101,7 @@ def test_batched_gris_spatial(room, neighbors):
 
 
 @pytest.mark.parametrize("count", [524287, 524288, 524289, 600001])
-def test_rays_beyond_one_per_lane(room, count):
+def test_rays_beyond_the_waves_in_flight(room, count):
     print(f"[gpu] rays {count}", flush=True)
     _, ds, osc = room
     rays = gpuhelp.random_rays(count, -0.9, 1.5, seed=count)

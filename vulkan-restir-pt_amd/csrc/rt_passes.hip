@@ -62,56 +62,28 @@ namespace {
 // ================================================================================================
 // Ray query test entry
 //
-// A wave takes `perWave` consecutive rays: a lane whose ray is done takes the wave's next one, so that the wave
-// stays full while its rays last. Lanes are refilled once kRefillLanes of them are idle, since a new ray's set-up
-// (six divisions) is issued for all of a refill's lanes at once. Up to 512k rays one ray per lane is faster (the
-// waves fit the device at once and none waits); at 1M random closest-hit rays two per lane take 329 against 338 us
-// on 20k triangles, 262 against 279 on 224k and 299 against 315 on 1.1M, where the fetches of the nodes bound both.
-constexpr int kRefillLanes = 32;
-constexpr uint32_t kTraceRounds = 2, kTraceWaves = 4096;
+// One ray per lane. Two per lane, the second taken once half the wave is idle, suits random rays only: they fill
+// lanes that would wait for the wave's longest ray, but rays of neighbouring pixels, which end together, lose the
+// waves in flight and each other's nodes (1M closest-hit rays on 1.1M triangles: random 294 us with two per lane and
+// 309 with one, a camera's 184 and 112; 4M: random 803 and 896, a camera's 423 and 298).
 template <bool kCount, bool kAny>
 __global__ __launch_bounds__(kTileThreads, RT_WAVES_TRACE) void k_trace_rays(DevScene S, const float* __restrict__ rays8, uint32_t n,
-                                                             uint32_t perWave, int skipLights, float* t, float* bary2,
+                                                             int skipLights, float* t, float* bary2,
                                                              uint32_t* inst, uint32_t* prim, TraceCounters* ctr) {
     __shared__ StackLDS<kTileThreads> stk;
+    const uint32_t i = blockIdx.x * kTileThreads + threadIdx.x;
+    if (i >= n) return;
     const TStack st = laneStack(stk);
-    StackSpill spill;
-    WalkWork work{0, 0};
-    unsigned long long rays = 0;
-    Walk w;
-    w.cur = RT_EMPTY;
-    Isec h;
-    uint32_t next = blockIdx.x * perWave;  // wave-uniform: the first ray not taken yet
-    const uint32_t end = min(n, next + perWave);
-    uint32_t ray = n;                      // this lane's ray, n: none
-    for (;;) {
-        // idle lanes: the finished ray's result, then the next ray
-        if (w.cur == RT_EMPTY && ray < n) {
-            const bool hit = h.inst != RT_INVALID_HIT;
-            if (kAny) {
-                inst[ray] = hit ? 1u : 0u; prim[ray] = 0; t[ray] = 0.0f; bary2[2 * (size_t)ray] = 0.0f; bary2[2 * (size_t)ray + 1] = 0.0f;
-            } else {
-                t[ray] = hit ? w.tBest : 0.0f; bary2[2 * (size_t)ray] = hit ? h.b1 : 0.0f; bary2[2 * (size_t)ray + 1] = hit ? h.b2 : 0.0f;
-                inst[ray] = h.inst; prim[ray] = hit ? h.prim : 0u;
-            }
-            ray = n;
-        }
-        const unsigned long long idle = __ballot(w.cur == RT_EMPTY);
-        if (next >= end && idle == __ballot(true)) break;
-        if (w.cur == RT_EMPTY) {
-            const uint32_t i = next + (uint32_t)__popcll(idle & ((1ull << threadIdx.x) - 1ull));
-            if (i < end) {
-                const float* q = rays8 + 8 * (size_t)i;
-                startWalk(S, w, mk3(q[0], q[1], q[2]), mk3(q[3], q[4], q[5]), q[6], q[7]);
-                h.inst = RT_INVALID_HIT;
-                ray = i;
-                if (kCount && S.numPrims != 0u) rays++;
-            }
-        }
-        next = min(end, next + (uint32_t)__popcll(idle));
-        walk<kAny, kCount, true>(S, w, !kAny && skipLights != 0, st, spill, next < end ? kTileThreads - kRefillLanes + 1 : 1, h, work);
+    const float* q = rays8 + 8 * (size_t)i;
+    const f3 o = mk3(q[0], q[1], q[2]), d = mk3(q[3], q[4], q[5]);
+    if (kAny) {
+        const bool occ = traceShadow<kCount>(S, st, o, q[6], d, q[7], ctr);
+        inst[i] = occ ? 1u : 0u; prim[i] = 0; t[i] = 0.0f; bary2[2 * (size_t)i] = 0.0f; bary2[2 * (size_t)i + 1] = 0.0f;
+    } else {
+        float th;
+        const Isec h = traceClosestHit<kCount>(S, st, o, q[6], d, q[7], ctr, skipLights != 0, &th);
+        t[i] = th; bary2[2 * (size_t)i] = h.b1; bary2[2 * (size_t)i + 1] = h.b2; inst[i] = h.inst; prim[i] = h.prim;
     }
-    if (kCount) countWork(ctr, work, rays);
 }
 
 // ================================================================================================
@@ -1896,15 +1868,11 @@ namespace rti {
 hipError_t launchTraceRays(const rt_device_scene* s, const float* rays8, uint32_t n, int mode, int skipLights, float* t,
                            float* bary2, uint32_t* inst, uint32_t* prim, hipStream_t stream) {
     if (n == 0) return hipSuccess;
-    // rays of one wave: one per lane until the waves would not fit the device at once, then up to
-    // kTraceRounds per lane
-    const uint32_t rounds = std::max(1u, std::min(kTraceRounds, n / (kTileThreads * kTraceWaves)));
-    const uint32_t perWave = kTileThreads * rounds;
-    const dim3 grid((unsigned)(((uint64_t)n + perWave - 1) / perWave));
+    const dim3 grid((n + kTileThreads - 1) / kTileThreads);
     TraceCounters* ctr = gCountersEnabled ? counterBuffer() : nullptr;
     const auto kernel = gCountersEnabled ? (mode == 1 ? k_trace_rays<true, true> : k_trace_rays<true, false>)
                                          : (mode == 1 ? k_trace_rays<false, true> : k_trace_rays<false, false>);
-    (void)launch(kernel, grid, kTileThreads, stream, s->dev, rays8, n, perWave, skipLights, t, bary2, inst, prim, ctr);
+    (void)launch(kernel, grid, kTileThreads, stream, s->dev, rays8, n, skipLights, t, bary2, inst, prim, ctr);
     return hipGetLastError();
 }
 
