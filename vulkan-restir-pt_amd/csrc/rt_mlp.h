@@ -138,36 +138,23 @@ RT_DEV void addFeature(float& f0, float& f1, float wt, uint32_t p) {
     f0 = f0 + wt * (float)a;
     f1 = f1 + wt * (float)b;
 }
-// The gathers bound the encoding: a lane's corners lie in cache lines of their own. The two corners neighbouring in
-// x are neighbours in a dense level's table, and for an even x an aligned pair in a hashed one's (the hash only
-// flips their lowest bit), so they are read as one 8-byte load there.
-// (300k points: 186 -> 172 us. The training kernel, at one wave per SIMD, reads all corners singly: 137 us with
-// pairs, 119 without, since it waits for the odd x's second loads.)
-struct __attribute__((packed, aligned(4))) FeaturePair { uint32_t a, b; };
-template <bool kPairs>
+// The gathers bound the encoding: a lane's corners lie in cache lines of their own. Two corners are indexed and then
+// read together, since the index's branch (dense or hashed level) holds up the reads behind it (300k points, tables
+// of 2^19 entries: 157 us, 176 corner by corner). One 8-byte read for two corners adjacent in memory is no gain: an
+// odd x needs a third read in a hashed level and waits for it (1M points: 482 us with it and 485 without, but with
+// tables of 2^15 entries 308 and 242; the 1080p proposal refresh 199 and 142, the learned target's 257 and 242).
 RT_DEV void encodeLevel(const MlpView& M, int l, float u, float v, float w, float& f0, float& f1) {
     uint32_t ci[3]; float fr[3];
     levelCell(M, l, u, v, w, ci, fr);
     f0 = 0.0f; f1 = 0.0f;
-    const bool dense = (M.denseMask >> l) & 1u;
-    const bool pair = dense || !(ci[0] & 1u);
     uint32_t p[8];
     float wt[8];
 #pragma unroll
     for (int c = 0; c < 8; c += 2) {
         const Corner k0 = corner(M, l, ci, fr, c), k1 = corner(M, l, ci, fr, c + 1);
         wt[c] = k0.wt; wt[c + 1] = k1.wt;
-        if (!kPairs) {
-            p[c] = M.grid[k0.slot];
-            p[c + 1] = M.grid[k1.slot];
-            continue;
-        }
-        const uint32_t first = min(k0.slot, k1.slot);
-        const FeaturePair f = *reinterpret_cast<const FeaturePair*>(M.grid + (pair ? first : k0.slot & ~1u));
-        const bool second = pair ? k0.slot != first : (k0.slot & 1u) != 0u;
-        p[c] = second ? f.b : f.a;
-        p[c + 1] = second ? f.a : f.b;  // a pair's other corner
-        if (!pair) p[c + 1] = M.grid[k1.slot];
+        p[c] = M.grid[k0.slot];
+        p[c + 1] = M.grid[k1.slot];
     }
 #pragma unroll
     for (int c = 0; c < 8; c++) addFeature(f0, f1, wt[c], p[c]);
@@ -175,13 +162,12 @@ RT_DEV void encodeLevel(const MlpView& M, int l, float u, float v, float w, floa
 
 // B operands of layer 1 for this lane: k-step s holds features 8s + 4h + (0..3)
 // = levels 4s + 2h and 4s + 2h + 1 of sample (u, v, w), h = lane / 32.
-template <bool kPairs = true>
 RT_DEV void encodeLane(const MlpView& M, uint32_t h, float u, float v, float w, h4 enc[4]) {
 #pragma unroll
     for (int s = 0; s < 4; s++) {
         float a0, a1, b0, b1;
-        encodeLevel<kPairs>(M, 4 * s + 2 * (int)h, u, v, w, a0, a1);
-        encodeLevel<kPairs>(M, 4 * s + 2 * (int)h + 1, u, v, w, b0, b1);
+        encodeLevel(M, 4 * s + 2 * (int)h, u, v, w, a0, a1);
+        encodeLevel(M, 4 * s + 2 * (int)h + 1, u, v, w, b0, b1);
         enc[s][0] = (_Float16)a0; enc[s][1] = (_Float16)a1;
         enc[s][2] = (_Float16)b0; enc[s][3] = (_Float16)b1;
     }

@@ -80,8 +80,8 @@ __device__ __forceinline__ void loadWeightsLDS(_Float16* sW, const _Float16* w) 
 
 // ---- inference ------------------------------------------------------------------------------
 // Radiance network: exp-activated RGB per sample. Proposal network: its 32 raw outputs per sample.
-// Held to four waves per SIMD (128 VGPRs): the gathers' latency bounds it (300k points: 172 us at the three waves of
-// its own allocation, 158 at four, 254 at five, where it spills).
+// Held to four waves per SIMD (128 VGPRs): the gathers' latency bounds it (300k points: 171 us at the three waves of
+// its own allocation, 157 at four; at five it spills).
 template <int kO>
 __global__ __launch_bounds__(64 * kInferWaves, 4) void k_mlp_infer(MlpView M, const float* __restrict__ pos, uint32_t n,
                                                                 float* __restrict__ out) {
@@ -240,7 +240,7 @@ __global__ __launch_bounds__(64) void k_mlp_train(MlpView M, const float* __rest
             valid = s < n && isfinite(y[3]) && y[3] > 0.0f && isfinite(y[0]) && isfinite(y[1]) && isfinite(y[2]) &&
                     invMean > 0.0f;
         h4 enc[4];
-        encodeLane<false>(M, (uint32_t)h, u, v, w, enc);
+        encodeLane(M, (uint32_t)h, u, v, w, enc);
         Fwd F;
         forwardTileT<kO>(L.w, lane, enc, F);
 
