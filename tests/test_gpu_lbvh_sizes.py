@@ -15,7 +15,8 @@ from test_gpu_traversal import light_scene  # noqa: E402
 rt = gpuhelp.rt
 
 
-@pytest.mark.parametrize("n", [2, 3, 1023, 1024, 1025, 4095, 4096, 4097, 8191, 262144, 262145, 524289])
+@pytest.mark.parametrize("n", [2, 3, 1023, 1024, 1025, 4095, 4096, 4097, 8191, 131072, 131073, 262144, 262145, 524288, 524289,
+                               786432, 786433])
 def test_build_matches_oracle(n):
     print(f"[gpu] lbvh {n}", flush=True)
     g = np.random.default_rng(n)

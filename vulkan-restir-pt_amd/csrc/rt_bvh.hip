@@ -166,10 +166,12 @@ __device__ __forceinline__ uint32_t blockExclusiveScan(uint32_t v, uint32_t* tot
 }
 
 // 4. radix sort, in tiles of 256 kI keys. A workgroup goes through its tile in kI rounds of barriers, so a sort of few
-// keys is faster over many small tiles: at 100k keys a pass's scatter takes 16.5 us with kI = 16 (25 workgroups), 5.4
-// with kI = 2, the whole build 354 -> 188 us.
+// keys is faster over many small tiles, one of many over few, whose histograms are less to scan. Whole build in us with
+// kI = 2, 4, 16: 65k keys 173, 181, 239; 131k 196, 199, 257; 197k 237, 228, 283; 524k 369, 341, 384; 786k 471, 410, 426;
+// 1.05M 557, 492, 472; 2.1M 965, 864, 777. The lines lie where the faster one changes.
+// k_radix_sort_small's line is its LDS (48 KB of pairs): 4096 keys take 130 us with it and 145 without, 1000 59 and 105.
 constexpr uint32_t kSmallSort = 4096;  // up to which one workgroup sorts in LDS (k_radix_sort_small)
-inline int radixItems(uint32_t n) { return n <= (1u << 18) ? 2 : (n <= (1u << 20) ? 4 : 16); }
+inline int radixItems(uint32_t n) { return n <= (1u << 17) ? 2 : (n <= (3u << 18) ? 4 : 16); }
 inline uint32_t radixTiles(uint32_t n) {
     const uint32_t tile = (uint32_t)kBlock * (uint32_t)radixItems(n);
     return n / tile + (n % tile ? 1u : 0u);
@@ -471,7 +473,8 @@ __device__ __forceinline__ uint32_t mergeNode(const float* nf, const uint32_t* h
 // A workgroup's time is its threads' climbs, one leaf after the other, each a chain of dependent fetches a level:
 // 1024 leaves a workgroup (one a thread) up to 512k primitives, 4096 beyond, where the top part, which one workgroup
 // finishes, would grow too long (100k primitives: 79 us over 25 workgroups of 4096 leaves, 23 over 98 of 1024; the
-// top part 47 -> 53 us).
+// top part 47 -> 53 us). Whole build in us with 1024 and 4096: 131k 196, 239; 393k 309, 325; 524k 339, 342; 786k 455,
+// 414; 2.1M 957, 779.
 constexpr uint32_t kRefitThreads = 1024;
 constexpr uint32_t kRefitLeaves = 4096;  // at most, per workgroup
 inline int refitShift(uint32_t n) { return n <= (1u << 19) ? 10 : 12; }
