@@ -319,8 +319,9 @@ RT_DEV void walk(const DevScene& S, Walk& w, bool skipLights, TStack st, StackSp
             const int n = (int)h0 + (int)h1 + (int)h2 + (int)h3;
             uint32_t key[4];  // of c3, c2, c1, c0 once ordered
             // Where tmin is a constant, i.e. everywhere but in ray queries and camera rays, the second order is not
-            // compiled. (1M rays from 1e-4: 324 us with both orders, 324 with the first alone.)
-            if (r.tmin > 0.0f) {
+            // compiled. (1M random rays on 1.1M triangles: 316 us from tmin = 1e-4, 311 with the first order alone; 354
+            // from tmin = 0.)
+            if (__builtin_expect(r.tmin > 0.0f, 1)) {
                 int k0 = pushKey(h0, t0, c0), k1 = pushKey(h1, t1, c1), k2 = pushKey(h2, t2, c2), k3 = pushKey(h3, t3, c3);
                 order4(k3, c3, k2, c2, k1, c1, k0, c0);
                 key[0] = ~(uint32_t)k3; key[1] = ~(uint32_t)k2; key[2] = ~(uint32_t)k1; key[3] = ~(uint32_t)k0;

@@ -1239,8 +1239,9 @@ __global__ __launch_bounds__(kTileThreads, kUnbiased ? RT_WAVES_SPATIAL_UB : RT_
 // not, so only the counting build traces that ray. Bound by the instructions of divergent traversal: one merge after
 // another runs at 16 of 64 lanes. The 1080p terrain frame takes 3.83 ms with this kernel and 4.04 without it, a 64x64
 // view of the box room 0.64 and 0.69, sixteen views in one batch 5.17 and 5.36. Its 12.4 KB of LDS let 12 waves share
-// a compute unit, hence 3 waves per SIMD: registers for 4 (more spilling, no more waves) give 3.93 ms. A fourth
-// neighbour's rays and weights would cost another of those waves, so more neighbours go to k_gris_spatial.
+// a compute unit, hence 3 waves per SIMD: registers for 4 (more spilling, no more waves) give 3.93 ms. The pool holds
+// every ray that kPoolNeighbors neighbours can ask for; it is not traced when full, so more neighbours go to
+// k_gris_spatial.
 constexpr uint32_t kPoolNeighbors = 3;
 struct SpatialPool {
     VisibilityPool<kPoolNeighbors * kTileThreads, true> rays;
