@@ -97,20 +97,21 @@ RT_DEV bool unpackGB(f4 dn, uint2 am, GPix& p) {
 }
 
 // ---- traversal wrappers (ray_query.glsl:6-70) ------------------------------------------------
-template <bool kCount, bool kCull = true>
+// kAnyTmin: tmin may be zero or negative; without it it must be positive (RT_MIN_RAY).
+template <bool kCount, bool kCull = true, bool kAnyTmin = false>
 RT_DEV Isec traceClosestHit(const DevScene& S, TStack st, f3 o, float tmin, f3 d, float tmax, TraceCounters* ctr,
                             bool skipLights = false, float* tOut = nullptr) {
     Isec h; h.b1 = 0.0f; h.b2 = 0.0f; h.inst = RT_INVALID_HIT; h.prim = 0;
     float tBest = tmax;
-    bool hit = traverse<false, kCount, kCull>(S, o, d, tmin, skipLights, st, tBest, h, ctr);
+    bool hit = traverse<false, kCount, kCull, kAnyTmin>(S, o, d, tmin, skipLights, st, tBest, h, ctr);
     if (!hit) { h.inst = RT_INVALID_HIT; h.b1 = 0.0f; h.b2 = 0.0f; h.prim = 0; }
     if (tOut) *tOut = hit ? tBest : 0.0f;
     return h;
 }
-template <bool kCount>
+template <bool kCount, bool kAnyTmin = false>
 RT_DEV bool traceShadow(const DevScene& S, TStack st, f3 o, float tmin, f3 d, float tmax, TraceCounters* ctr) {
     Isec h; float tBest = tmax;
-    return traverse<true, kCount>(S, o, d, tmin, false, st, tBest, h, ctr);
+    return traverse<true, kCount, true, kAnyTmin>(S, o, d, tmin, false, st, tBest, h, ctr);
 }
 template <bool kCount>
 RT_DEV bool traceVisibility(const DevScene& S, TStack st, f3 from, f3 to, TraceCounters* ctr) {

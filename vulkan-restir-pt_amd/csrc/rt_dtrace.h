@@ -235,8 +235,9 @@ RT_DEV void startWalk(const DevScene& S, Walk& w, f3 o, f3 d, float tmin, float 
 // Walks the lanes' rays until fewer than minBusy of the wave's (converged) lanes are busy. kAny: a lane stops at
 // its first hit. hit.inst is set on a hit and is the caller's to initialise. kCull: closest-hit queries drop
 // popped nodes beyond the closest hit (the result is the same either way; the reuse passes' replays, which rarely
-// pop such nodes, leave it off to save registers).
-template <bool kAny, bool kCount, bool kCull, int kStackWords = 2 * RT_LDS_STACK>
+// pop such nodes, leave it off to save registers). kAnyTmin: the rays' tmin may be zero or negative; without it they
+// must be positive.
+template <bool kAny, bool kCount, bool kCull, int kStackWords = 2 * RT_LDS_STACK, bool kAnyTmin = false>
 RT_DEV void walk(const DevScene& S, Walk& w, bool skipLights, TStack st, StackSpill& spill, int minBusy, Isec& hit,
                  WalkWork& work) {
     constexpr bool kKeep = kCull && !kAny;  // keys kept on the stack
@@ -318,10 +319,7 @@ RT_DEV void walk(const DevScene& S, Walk& w, bool skipLights, TStack st, StackSp
             }
             const int n = (int)h0 + (int)h1 + (int)h2 + (int)h3;
             uint32_t key[4];  // of c3, c2, c1, c0 once ordered
-            // Where tmin is a constant, i.e. everywhere but in ray queries and camera rays, the second order is not
-            // compiled. (1M random rays on 1.1M triangles: 316 us from tmin = 1e-4, 311 with the first order alone; 354
-            // from tmin = 0.)
-            if (__builtin_expect(r.tmin > 0.0f, 1)) {
+            if (!kAnyTmin || r.tmin > 0.0f) {
                 int k0 = pushKey(h0, t0, c0), k1 = pushKey(h1, t1, c1), k2 = pushKey(h2, t2, c2), k3 = pushKey(h3, t3, c3);
                 order4(k3, c3, k2, c2, k1, c1, k0, c0);
                 key[0] = ~(uint32_t)k3; key[1] = ~(uint32_t)k2; key[2] = ~(uint32_t)k1; key[3] = ~(uint32_t)k0;
@@ -377,7 +375,7 @@ RT_DEV void countWork(TraceCounters* ctr, const WalkWork& work, unsigned long lo
 }
 
 // One ray per lane, to the end.
-template <bool kAny, bool kCount, bool kCull = true>
+template <bool kAny, bool kCount, bool kCull = true, bool kAnyTmin = false>
 RT_DEV bool traverse(const DevScene& S, f3 o, f3 d, float tmin, bool skipLights, TStack st, float& tBest, Isec& hit,
                      TraceCounters* ctr) {
     StackSpill spill;
@@ -385,7 +383,7 @@ RT_DEV bool traverse(const DevScene& S, f3 o, f3 d, float tmin, bool skipLights,
     Walk w;
     startWalk(S, w, o, d, tmin, tBest);
     hit.inst = RT_EMPTY;
-    walk<kAny, kCount, kCull>(S, w, skipLights, st, spill, 1, hit, work);
+    walk<kAny, kCount, kCull, 2 * RT_LDS_STACK, kAnyTmin>(S, w, skipLights, st, spill, 1, hit, work);
     tBest = w.tBest;
     if (kCount && S.numPrims != 0u) countWork(ctr, work, 1ull);
     return hit.inst != RT_EMPTY;
